@@ -70,6 +70,44 @@ def test_quantizer_power_of_two_scale_edges(lib):
     assert float(scales[0, 0, 7]) == 2.0 ** -126 and float(scales[0, 0, 8]) == 1.0
 
 
+@pytest.mark.parametrize("order", ["sorted", "shuffled"])
+def test_quantizer_every_finite_value(lib, order):
+    """Every finite bf16 value, in blocks of like magnitudes (every scale exponent) and mixed
+    (most codes subnormal or zero), with a partial last block; bit-exact against the oracle."""
+    from lbw_amd import quantize_kv_fp8
+    bits = torch.arange(65536, dtype=torch.int32)
+    bits = bits[(bits & 0x7f80) != 0x7f80]                    # no infinities, no NaNs
+    bits = bits[torch.argsort(bits & 0x7fff, stable=True)]    # by magnitude
+    if order == "shuffled":
+        bits = bits[torch.randperm(bits.numel(), generator=torch.Generator().manual_seed(5))]
+    x = bits.to(torch.int16).view(torch.bfloat16).view(1, -1, 1, 128)
+    x = torch.cat([x, x[:, :37] * 0.5], dim=1).repeat(1, 1, 2, 1)
+    q = quantize_kv_fp8(x.to(DEV))
+    codes, scales = O.quantize_kv_fp8(x.float())
+    assert torch.equal(q.scales.cpu(), scales) and torch.equal(q.codes.cpu(), codes)
+
+
+def test_quantizer_infinities_and_nans(lib):
+    """A block with infinities or NaNs: NaNs take no part in the scale, both get a NaN code with
+    their sign, the block's other values theirs, and other blocks are not touched."""
+    from lbw_amd import quantize_kv_fp8
+    g = torch.Generator().manual_seed(11)
+    x = torch.randn(1, 256, 2, 128, generator=g).to(torch.bfloat16)
+    x[0, 70, 0, 3], x[0, 90, 0, 100] = float("nan"), -float("nan")
+    x[0, 130, 1, 7], x[0, 131, 1, 8] = float("inf"), -float("inf")
+    x[0, 192:, 0] = float("nan")                               # nothing but NaNs: scale 1
+    q = quantize_kv_fp8(x.to(DEV))
+    t = x.float().view(1, 4, 64, 2, 128)
+    amax = torch.where(t.isnan(), torch.zeros(()), t.abs()).amax(dim=(2, 4))
+    amax = amax.clamp(max=2.0 ** 128 - 2.0 ** 104)             # an infinity: the exponent above
+    k = torch.frexp(amax / 448.0)[1]
+    k = torch.where(torch.frexp(amax / 448.0)[0] == 0.5, k - 1, k)
+    scale = torch.where(amax > 0, torch.ldexp(torch.ones_like(amax), k), torch.ones_like(amax))
+    assert torch.equal(q.scales.cpu(), scale.permute(0, 2, 1))
+    codes = (t / scale[:, :, None, :, None]).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(q.codes.cpu(), codes.view(1, 256, 2, 128))
+
+
 @pytest.mark.parametrize("Lq,H,lk,window", [(300, 2, 2000, None), (100, 3, 777, (13, 700))])
 def test_fp8_attention_cosine(lib, Lq, H, lk, window):
     from lbw_amd import attention_fp8kv, quantize_kv_fp8
