@@ -166,6 +166,19 @@ __device__ __forceinline__ int take_item(uint32_t* q, uint32_t U, uint32_t S, ui
   return -1;
 }
 
+// The item of workgroup i without queues (the items fit the CUs at once, or the caller gave no
+// workspace): XCD i % 8 takes an eighth of the items in (batch x head, piece, q-tile) order, so
+// that no XCD has more than its CUs when the items fit the chip, and the q-tiles that read the
+// same keys stay together. -1: no item.
+__device__ __forceinline__ int static_item(uint32_t U, uint32_t S, uint32_t nq, uint32_t i) {
+  const uint32_t N = U * S;
+  uint32_t st, n;
+  xcd_units(N, i & 7u, st, n);
+  if ((i >> 3) >= n) return -1;
+  const uint32_t o = st + (i >> 3), bh = o / (S * nq), r = o % (S * nq);
+  return (int)((r / nq) * U + bh * nq + r % nq);
+}
+
 __global__ void __launch_bounds__(256) attn_queue_reset_kernel(uint32_t* q, int n) {
   for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) q[i] = 0u;
 }
@@ -275,7 +288,7 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
   const int l32 = lane & 31;
 
   // ---- work item (piece, unit). With a work queue the items are handed out at run time;
-  // without, workgroup i takes item i / 8 of XCD i % 8 (workgroups reach the XCDs round-robin).
+  // without, workgroup i takes a fixed one (static_item; workgroups reach the XCDs round-robin).
   const uint32_t U = (uint32_t)a.n_qtiles * a.H * a.B;
   uint32_t id;
   {
@@ -284,10 +297,7 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
       if (threadIdx.x == 0) s_item = take_item(a.queue, U, a.splits, blockIdx.x & 7u);
       __syncthreads();
     } else if (threadIdx.x == 0) {
-      uint32_t st, n;
-      xcd_units(U, blockIdx.x & 7u, st, n);
-      const uint32_t j = blockIdx.x >> 3;
-      s_item = j < a.splits * n ? (int)((j / n) * U + st + j % n) : -1;
+      s_item = static_item(U, a.splits, a.n_qtiles, blockIdx.x);
     }
     __syncthreads();
     const int item = s_item;
@@ -1239,12 +1249,12 @@ static hipError_t launch(const AttnKernelArgs& a, hipStream_t stream) {
       hipFuncAttributeMaxDynamicSharedMemorySize, LDS_B);
   if (attr != hipSuccess) return attr;
   const uint32_t U = (uint32_t)a.n_qtiles * a.H * a.B;
-  const uint32_t per_xcd = a.splits * ((U + 7u) / 8u);  // items of the largest XCD share
-  uint32_t nwg = 8u * per_xcd;
+  uint32_t nwg = 8u * ((a.splits * U + 7u) / 8u);  // static items: an eighth per XCD
   if (a.queue != nullptr) {
     // spare workgroups, 1/16 of an XCD's share (at least one each): enough for the measured
     // spread of XCD speeds (a few percent)
-    nwg += 8u * ((per_xcd + 15u) / 16u);
+    const uint32_t per_xcd = a.splits * ((U + 7u) / 8u);  // items of the largest XCD share
+    nwg = 8u * (per_xcd + (per_xcd + 15u) / 16u);
     // the 8 queue counters and, for the in-kernel merge, the U arrival counters after them
     const int n = 8 + (a.merge_cnt != nullptr ? (int)U : 0);
     hipLaunchKernelGGL(attn_queue_reset_kernel, dim3((n + 255) / 256 < 64 ? (n + 255) / 256 : 64),

@@ -55,16 +55,21 @@ int num_cus() {
   return cache[dev];
 }
 
-// Estimated run time, in tile steps, of a launch with s KV splits: greedy list scheduling of
-// the workgroups in dispatch order (q-tile fastest, then split, then batch x head) over the
-// CUs, one workgroup per CU. A workgroup costs its tile count times (0.3 + 0.7 * its share of
-// active query waves); each split beyond the first adds 3 % (partials written and merged).
-// The constants are fitted to measured gfx950 times of the 1.3B/14B chunk shapes.
+// Estimated run time, in tile steps (1.5 us), of a launch with s KV splits: greedy list
+// scheduling of the workgroups in dispatch order (q-tile fastest, then split, then batch x head)
+// over the CUs, one workgroup per CU. A workgroup costs its tile count times (0.3 + 0.7 * its
+// share of active query waves), and a fixed part: taking the item, Q and the first tiles, the
+// output and the next workgroup's start, 5 tile steps, or 10 when its keys are a piece of the
+// unit's (partials written, and a share of their merge); 1 % per further piece decides between
+// near equals. Fitted to measured gfx950 times, in
+// us, of 1, 2, 3, .. pieces: 40 heads x 3600 q x 3600 keys 267, 290, 325; 10 x 3600 x 46800 850,
+// 969, 745, 790, 725, 773; 12 x 1560 x 4680 100, 70, 60, 82; 12 x 4680 x 14040 343, 364, 373.
 double split_cost(int64_t bh, int lq, int bm, int64_t ntiles, int s, int cus) {
   const int nq = (lq + bm - 1) / bm;
   const int tail_q = lq - (nq - 1) * bm;                  // queries in the last q-tile
   const double tail_w = (double)((tail_q + 31) / 32) / (bm / 32);
   const int64_t per = (ntiles + s - 1) / s;
+  const double fixed = s == 1 ? 5.0 : 10.0;
   std::priority_queue<double, std::vector<double>, std::greater<double>> cu;
   for (int i = 0; i < cus; ++i) cu.push(0.0);
   for (int64_t g = 0; g < bh; ++g)
@@ -75,15 +80,17 @@ double split_cost(int64_t bh, int lq, int bm, int64_t ntiles, int s, int cus) {
         const double w = qt + 1 < nq ? 1.0 : tail_w;
         const double t = cu.top();
         cu.pop();
-        cu.push(t + tiles * (0.3 + 0.7 * w));
+        cu.push(t + tiles * (0.3 + 0.7 * w) + fixed);
       }
     }
   double span = 0.0;
   while (!cu.empty()) { span = cu.top(); cu.pop(); }
-  return span * (1.0 + 0.03 * (s - 1));
+  return span * (1.0 + 0.01 * (s - 1));
 }
 
-// Number of KV splits (1..8) with the lowest estimated time; decisions are cached per shape.
+// Number of KV splits with the lowest estimated time, pieces of 4 tiles at least; up to 8, or up
+// to 16 while every piece has a CU of its own (5 heads x 1001 q x 10000 keys, 20 units: 8 pieces
+// 43 us, 12 40 us). Decisions are cached per shape.
 int choose_splits(int64_t bh, int lq, int bm, int64_t ntiles, int cus) {
   struct Entry { int64_t bh, ntiles; int lq, cus, splits; };
   static std::mutex mu;
@@ -100,7 +107,7 @@ int choose_splits(int64_t bh, int lq, int bm, int64_t ntiles, int cus) {
   const int64_t nq = (lq + bm - 1) / bm;
   if (bh * nq * 8 <= 200000) {  // keep the simulation cheap; huge launches need no split
     double best = split_cost(bh, lq, bm, ntiles, 1, cus);
-    for (int s = 2; s <= 8 && ntiles / s >= 8; ++s) {
+    for (int s = 2; s <= (bh * nq * s <= cus ? 16 : 8) && ntiles / s >= 4; ++s) {
       const double c = split_cost(bh, lq, bm, ntiles, s, cus);
       if (c < best) { best = c; best_s = s; }
     }
@@ -115,12 +122,16 @@ int choose_splits(int64_t bh, int lq, int bm, int64_t ntiles, int cus) {
 constexpr size_t kQueueBytes = 256;  // 8 work-queue counters, padded
 
 // Split calls of up to this many pieces merge their partials in the attention kernel (the last
-// piece of each unit); more pieces run the separate merge kernel.
+// piece of each unit); more pieces run the separate merge kernel. So do calls whose items all run
+// at once, one per CU (one_round): a unit's last piece would merge alone at the end of the launch
+// (7-11 us) what the merge kernel spreads over the chip, and with no counters to clear and no
+// items to hand out they need no reset launch and no queues.
 constexpr int kMaxFusedSplits = 8;
 
 struct Plan {
   AttnKernelArgs a;
   int splits;
+  bool one_round;     // every work item has a CU of its own: fixed items, no queues
   bool fused_merge;   // the pieces merge in-kernel (no merge launch)
   size_t part_bytes;  // split partials
   size_t queue_off;   // work-queue counters
@@ -259,8 +270,9 @@ int make_plan(const lbw_attn_params* p, bool fp8, Plan* plan) {
   // pieces merge in-kernel) one arrival counter per unit]
   plan->part_bytes = splits > 1 ? (size_t)splits * a.B * a.H * a.Lq * (p->head_dim + 2) * sizeof(float) : 0;
   plan->queue_off = (plan->part_bytes + 255) & ~(size_t)255;
-  plan->fused_merge = splits > 1 && splits <= kMaxFusedSplits;
   const size_t units = (size_t)a.n_qtiles * a.H * a.B;
+  plan->one_round = units * splits <= (size_t)num_cus();
+  plan->fused_merge = splits > 1 && splits <= kMaxFusedSplits && !plan->one_round;
   const size_t cnt_bytes = (8 + (plan->fused_merge ? units : 0)) * sizeof(uint32_t);
   plan->ws_bytes = plan->queue_off + std::max(kQueueBytes, (cnt_bytes + 255) & ~(size_t)255);
   a.splits = splits;
@@ -317,7 +329,7 @@ int run_attention(const lbw_attn_params* p, bool fp8, void* ws, size_t ws_bytes,
     return LBW_OK;
   }
   const bool ws_ok = ws != nullptr && ws_bytes >= plan.ws_bytes && aligned16(ws);
-  if (ws_ok) {
+  if (ws_ok && !plan.one_round) {
     a.queue = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(ws) + plan.queue_off);
   }
   if (plan.splits > 1) {

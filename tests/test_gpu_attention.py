@@ -397,6 +397,28 @@ def test_split_pieces_merged_in_kernel(lib, splits):
     assert torch.equal(o32.to(torch.bfloat16), runs[0])
 
 
+@pytest.mark.parametrize("H,Lq,keys,splits", [
+    (8, 2048, 1100, 4),    # 256 items: a CU each on a 256-CU chip, no queues
+    (8, 2048, 1100, 5),    # 320 items: queues and the in-kernel merge
+    (5, 700, 1900, 12),    # more pieces than the in-kernel merge takes, uneven XCD shares
+    (3, 40, 1300, 16),     # one partial q-tile per head, more pieces than tiles need
+    (1, 33, 70, 0),        # one workgroup
+    (5, 600, 5000, 0),     # the host's own choice, more than 8 pieces
+])
+def test_items_in_one_round(lib, H, Lq, keys, splits):
+    """Calls whose work items all run at once take fixed items (no queues, no reset launch) and
+    the separate merge: parity with the oracle, repeated calls bit for bit equal."""
+    from lbw_amd import attention_segments
+    q, ks, vs = _case(1, Lq, H, [keys], seed=H + splits, gain=False)
+    segs = [(k.to(DEV), v.to(DEV)) for k, v in zip(ks, vs)]
+    qd = q.to(DEV)
+    runs = [attention_segments(qd, segs, num_splits=splits) for _ in range(3)]
+    torch.cuda.synchronize()
+    assert_parity(runs[0], O.attention_ref(q, torch.cat(ks, 1), torch.cat(vs, 1)))
+    for r in runs[1:]:
+        assert torch.equal(r, runs[0])
+
+
 def test_chain_state_is_one_running_triple(lib):
     """The chain state is one (O, m, l) triple merged call by call (the reference's running
     (O, -max, sum)): 20 calls -- more than one merge launch takes partials -- over 20 key
