@@ -261,6 +261,10 @@ __device__ void merge_unit(const AttnKernelArgs& a, int b, int h, int qt, int ro
 // FOLD: scale * log2(e) == 1, i.e. q already carries log2(e)/sqrt(d) (a pre-scaled q, as the
 // fused q/k kernel writes it): the QK chain starts from -m instead of 0, so the MFMA result is
 // already the exponent of p and the softmax needs no per-score FMA (see the step).
+// TRACK: the caller's partials, whose m is the row's true max: the running max is kept beside the
+// softmax (8 three-way maxima per step, off its path) and O and l move to it at the end. Deciding
+// the reference by it in every step, ahead of the exponentials, took 48.5 us against 45.3 at 12
+// heads x 1560 q x 1560 keys and 318 against 304 at 40 x 3600 x 3600.
 // SEGN = 1 or 2: that many KV segments (a flat cache's window; a cache and the current chunk),
 // no multiplicity bias and, for two, the same row strides: the tile copies are addressed by the
 // tile index (issue1, issue_raw1, issue_k81) instead of walked by the general cursor (SEGN 0).
@@ -431,7 +435,6 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
   const float mult_raw = sreg(a.mult_raw);
   // the call carries a multiplicity bias (mult_key >= 0: the sign of its high word)
   const int mult = sreg((int)(a.mult_key >> 32)) >= 0;
-  const float tau_raw = TAU / c;
 
   // DMA of the cursor's tile into a stage (2*NDMA x 16 B per lane); returns the tile's row
   // info (pack_rows). Full tiles use the per-segment lane offsets; in a partial
@@ -707,17 +710,13 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
 
     // Pipeline registers, double-buffered so that consecutive steps swap roles instead of
     // copying: S of the sub-block being softmaxed / being computed, P of the previous / current
-    // sub-block. `pend` / `alpha_p` (TRACK): an O rescale decided at the start of the previous
-    // step, applied at the start of the next one (after the PV MFMAs that still used the old
-    // reference). The other forms decide a move after the step's MFMAs and rescale O right in
-    // the redo branch, so the common path carries no rescale branch.
+    // sub-block. A move of the exponent reference is decided after the step's MFMAs and rescales
+    // O right in the redo branch, so the common path carries no rescale branch.
     floatx16 sA, sB, cinit;  // cinit (FOLD): -mref, the start of every QK chain
 #pragma unroll
     for (int r = 0; r < 16; ++r) { sA[r] = 0.0f; sB[r] = 0.0f; cinit[r] = 0.0f; }
     u32x4 pA[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
     u32x4 pB[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-    bool pend = false;
-    float alpha_p = 1.0f;
 
     // LDS fragments in flight: K of pair i in kf[i % KR], V in vf[i % VR]. The rings hold a
     // multiple of 8 slots' worth of indices (8 % KR == 0), so the last pairs of a step can read
@@ -802,9 +801,6 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
 #pragma unroll
         for (int i = 0; i < V_AHEAD; ++i) load_v(voff_c, i);
       }
-      if constexpr (TRACK) {
-        if (pend) scale_acc(oacc, alpha_p);
-      }
       if constexpr (BIAS) {
         // this lane's keys 32 kb + 8 g + 4 hl .. +3 (registers 4g .. 4g+3) of the tile being
         // softmaxed (stage KS for the first half's step, the stage before SN for the second's)
@@ -822,23 +818,11 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
       const int vlo = vrow & 0xff, vhi = (vrow >> 8) & 0xff, mrow = vrow >> 16;
       if (vrow != ROWS_FULL && (vlo > 32 * kb || vhi < 32 * kb + 32 || mrow < 32 * kb + 32))
         mask_scores(s_in, kb, vlo, vhi, hl, mrow, mult_raw);
-      // softmax, part 1 (TRACK): running max and exponent reference, decided before the
-      // exponentials (wave-uniform). Without TRACK the exponentials use the current reference
-      // and part 3 checks them afterwards.
-      bool move = false;
-      float alpha = 1.0f;
+      // TRACK: the row's true max besides, off the softmax's path (16 keys per lane; lanes l and
+      // l^32 hold the two halves of a query's keys and are joined at the end)
       if constexpr (TRACK) {
-        // lanes l and l^32 hold the same query's running max: fold it in before the exchange
-        float mx = m_true;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s_in[r]);
-        m_true = wave_max_xor32(mx);
-        // Every lane sees the same valid keys, so m_true is -inf in all lanes or in none, and
-        // a move never selects -inf.
-        move = __any(m_true > m_used + tau_raw);
-        const float m_new = move ? m_true : m_used;
-        alpha = fast_exp2((m_used - m_new) * c);
-        m_used = m_new;
+        for (int r = 0; r < 16; r += 2) m_true = fmaxf(fmaxf(m_true, s_in[r]), s_in[r + 1]);
       }
       // The reference starts at M_INIT, a finite stand-in for -inf, so no step needs an
       // infinity case: masked scores (-inf) give p = 0, and the first valid score moves it.
@@ -971,7 +955,7 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
           float d;  // the reference's move, log2 units
           if (mlim > 0.0f) {
             d = fmaxf(mx, 0.0f);
-            alpha = fast_exp2(-d);
+            const float alpha = fast_exp2(-d);
             // O (with this step's PV of the previous sub-block, at the old reference) and the
             // row sum move now
             scale_acc(oacc, alpha);
@@ -981,7 +965,6 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
             d = set ? mx : 0.0f;
             mlim = set ? P_LIMIT : -1.0f;
           }
-          move = true;
           mref += d;
           // s_out (the next sub-block, started from the old -mref in this step) moves too
 #pragma unroll
@@ -992,7 +975,7 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
           }
           ls = exps();
         }
-      } else if constexpr (!TRACK) {
+      } else {
         // P is packed in this block, not in the redo branch's successors
         asm volatile("" ::"v"(p_out[0]), "v"(p_out[1]), "v"(ls));
         // softmax, part 3: a row sum beyond 2^16 (or not finite) means some p outgrew the
@@ -1005,9 +988,8 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
           for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s_in[r]);
           mx = wave_max_xor32(mx);
           const float m_new = fmaxf(mx, m_used);
-          alpha = fast_exp2((m_used - m_new) * c);
+          const float alpha = fast_exp2((m_used - m_new) * c);
           m_used = m_new;
-          move = true;
           ca = -m_new * c;
           // O (with this step's PV of the previous sub-block, at the old reference) and the
           // row sum move now
@@ -1016,14 +998,10 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
           ls = exps();
         }
       }
-      // (TRACK decided its move before the exponentials; the other forms rescaled lsum in the
-      // redo branch, so their common path is one add)
-      if constexpr (TRACK) lsum = __builtin_fmaf(lsum, alpha, ls);
-      else lsum += ls;
+      lsum += ls;
       // keep the exponentials in this step's block (not sunk into the next one)
       asm volatile("" ::"v"(p_out[0]), "v"(p_out[1]), "v"(lsum));
-      pend = TRACK && move;  // (the other forms have rescaled O in the redo branch)
-      alpha_p = alpha;
+      if constexpr (TRACK) asm volatile("" ::"v"(m_true));
     };
 
     // Tile u lives in stage u % NSTAGE (K at stage*16 KB, V at V_BASE + stage*16 KB).
@@ -1093,7 +1071,6 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
 
     // drain: O += V^T P^T of the last sub-block (tile T-1 half 1, P in pA)
     if (wave_active) {
-      if (pend) scale_acc(oacc, alpha_p);
       const int vo = ((T - 1) % NSTAGE) * TILE_B + HALF_B;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -1154,12 +1131,13 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
     const bool norm32 = a.mode == kModeNormalized;
     float f = 1.0f;
     float m_out = -INFINITY;
+    const float m_row = TRACK ? wave_max_xor32(m_true) : 0.0f;
     if (norm32) {
       f = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     } else if (l_tot > 0.0f) {
       if constexpr (TRACK) {
-        f = fast_exp2((m_used - m_true) * c);
-        m_out = m_true * a.scale;
+        f = fast_exp2((m_used - m_row) * c);
+        m_out = m_row * a.scale;
       } else if constexpr (FOLD) {
         m_out = mref * a.scale;
       } else {
@@ -1283,9 +1261,10 @@ hipError_t launch_attn_fwd(const AttnKernelArgs& a, hipStream_t stream) {
     if (a.scale_log2 == 1.0f) return launch<false, false, true, 0, true>(a, stream);
     return launch<false, false, false, 0, true>(a, stream);
   }
-  if (a.track_max) return launch<false, true>(a, stream);
-  // a pre-scaled q (scale * log2(e) exactly 1 in fp32) takes the folded softmax
   const int segn = index_segments(a);
+  if (a.track_max) return segn == 1 ? launch<false, true, false, 1>(a, stream)
+                                    : launch<false, true>(a, stream);
+  // a pre-scaled q (scale * log2(e) exactly 1 in fp32) takes the folded softmax
   if (a.scale_log2 == 1.0f) {
     if (segn == 1) return launch<false, false, true, 1>(a, stream);
     if (segn == 2) return launch<false, false, true, 2>(a, stream);

@@ -12,7 +12,6 @@ namespace lbw {
 
 constexpr int D = 128;
 constexpr int BN = 64;
-constexpr float TAU = 8.0f;  // lazy-rescale threshold, log2 units
 constexpr float M_INIT = -1e30f;  // initial exponent reference (finite stand-in for -inf)
 constexpr float P_LIMIT = 65536.0f;  // largest per-lane row sum before the reference moves
 
