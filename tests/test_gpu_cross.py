@@ -58,6 +58,20 @@ def test_cross_matches_oracle(lib, B, Lq, H, L, lens):
     assert_parity(out, ref, "cross")
 
 
+@pytest.mark.parametrize("H,Lq", [(1, 250), (3, 500), (3, 700), (7, 520), (5, 3900), (51, 1300)])
+@pytest.mark.parametrize("L", [100, 400])
+def test_cross_rounds_below_and_above_the_grid(lib, H, Lq, L):
+    """Round counts (heads x ceil(Lq / 256)) of 1, 6, 9, 21, 80 and 306, not multiples of 8 for the
+    most part, so that the grid holds workgroups with no round (and, past the CUs, several per
+    workgroup), in the resident (100 keys) and the ring form (400): every row is written."""
+    from lbw_amd import cross_attention
+    q, k, v = _qkv(1, Lq, H, L, seed=Lq + L + H)
+    print(f"case H={H} Lq={Lq} L={L}", flush=True)
+    out = cross_attention(q.to(DEV), k.to(DEV), v.to(DEV))
+    assert_parity(out, O.attention_ref(q, k, v), "cross rounds")
+
+
+
 @pytest.mark.parametrize("H,Lq", [(40, 4680), (7, 1000)])
 def test_cross_rounds_across_workgroups_fp32(lib, H, Lq):
     """Many heads (rounds of one head spread over several workgroups, workgroups spanning two
