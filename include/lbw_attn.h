@@ -22,6 +22,7 @@
  *                          kernels/cross_dedup.py              cross_dedup_kernel
  *   lbw_attn_merge         wan/modules/attention.py:963-990    cte_merge
  *   lbw_attn_merge_partials wan/modules/attention.py:654-694   cte_call's chain state
+ *   lbw_attention_chain    wan/modules/attention.py:654-694    cte_call, one call of the chain
  *   lbw_qk_norm_rope       kernels/qk_post.py:404-413          qk_ss + qk_norm_rope
  *                          (caller wan/modules/model_fast.py:2596-2681 _qkv_post)
  *   lbw_kv_quant_fp8       no reference counterpart (new fp8-e4m3 KV cache)
@@ -182,6 +183,20 @@ int lbw_attn_merge_partials(int32_t n_parts, const float* const* part_o,
                             const float* const* part_m, const float* const* part_l, int32_t batch,
                             int32_t heads, int32_t lq, int32_t head_dim, float* out_o,
                             float* out_m, float* out_l, void* stream);
+
+/* One call of cte_call's chain (wan/modules/attention.py:654-694): attention over the params' KV
+ * segments joined with the running triple of the earlier calls (state_o [B, H, Lq, D], state_m and
+ * state_l [B, H, Lq], fp32, contiguous; all three NULL for a chain's first call). With part_o,
+ * part_m and part_l the new triple is written there (m the true row max; it must not overlap the
+ * state); without them the chain ends and `out` gets the normalised result. The results are those
+ * of lbw_attention_fwd's partials and lbw_attn_merge_partials / lbw_attn_merge up to fp32
+ * rounding; the call's keys may be cut into pieces that run side by side (num_splits: 0 = the
+ * host's choice, up to 15). The workspace holds the pieces' partials and, as for
+ * lbw_attention_fwd, backs one in-flight call. */
+size_t lbw_attention_chain_workspace_size(const lbw_attn_params* p, int32_t has_state);
+int lbw_attention_chain(const lbw_attn_params* p, const float* state_o, const float* state_m,
+                        const float* state_l, void* workspace, size_t workspace_bytes,
+                        void* stream);
 
 /* Fused q/k post-processing of one chunk (kernels/qk_post.py semantics, full-row RMSNorm):
  *   y = x + b (fp32); r = rsqrt(sum(y^2)/C + eps); t = bf16(y*r) * gamma (fp32);

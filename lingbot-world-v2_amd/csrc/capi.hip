@@ -365,6 +365,106 @@ int run_attention(const lbw_attn_params* p, bool fp8, void* ws, size_t ws_bytes,
   return LBW_OK;
 }
 
+// One call of the chain: its plan on top of the plain one. The call's keys are cut into pieces
+// while every piece still has a CU of its own (a call over one cached chunk has too few q-tiles to
+// fill the chip), and one merge launch joins the pieces and the earlier calls' state.
+struct ChainPlan {
+  Plan plan;
+  bool plain;         // no state, normalised output: the plain attention call
+  bool direct;        // one piece, no state: the kernel writes the caller's triple itself
+};
+
+int make_chain_plan(const lbw_attn_params* p, bool state, ChainPlan* c) {
+  if (p == nullptr) return fail(LBW_ERR_INVALID, "params is NULL");
+  lbw_attn_params one = *p;
+  one.num_splits = 1;
+  const bool triple = p->part_o != nullptr;
+  c->plain = !state && !triple;
+  int rc = make_plan(c->plain ? p : &one, false, &c->plan);
+  if (rc != LBW_OK || c->plain) return rc;
+  AttnKernelArgs& a = c->plan.a;
+  if (a.key_bias != nullptr) return fail(LBW_ERR_UNSUPPORTED, "key_bias: not in a chained call");
+  const int64_t units = (int64_t)a.n_qtiles * a.H * a.B;
+  // 1..15 pieces (the merge takes 16 partials). 12 heads x 1560 q x 1560 keys (84 units), a call in
+  // the middle of a chain with its merge: 54.5 us in one piece, 35.4 in three; 5 x 3600 x 3600 (75
+  // units) 98.7 and 50.3
+  int splits = p->num_splits > 15 ? 15 : p->num_splits;
+  if (splits <= 0) {
+    const int64_t ntiles = (a.hi - a.lo + attn_block_n() - 1) / attn_block_n();
+    splits = 1;
+    if (units > 0 && 2 * units <= num_cus()) {
+      splits = choose_splits((int64_t)a.H * a.B, p->lq, attn_block_m(), ntiles, num_cus());
+      splits = (int)std::min<int64_t>(std::min(splits, 15), num_cus() / units);
+    }
+  }
+  c->direct = splits == 1 && !state;
+  Plan& plan = c->plan;
+  plan.splits = a.splits = splits;
+  plan.one_round = units * splits <= num_cus();
+  plan.fused_merge = false;
+  plan.part_bytes = c->direct ? 0 : (size_t)splits * a.B * a.H * a.Lq * (p->head_dim + 2) * sizeof(float);
+  plan.queue_off = (plan.part_bytes + 255) & ~(size_t)255;
+  plan.ws_bytes = plan.queue_off + kQueueBytes;
+  return LBW_OK;
+}
+
+int run_chain(const lbw_attn_params* p, const float* so, const float* sm, const float* sl, void* ws,
+              size_t ws_bytes, void* stream) {
+  const bool state = so != nullptr || sm != nullptr || sl != nullptr;
+  if (state && (so == nullptr || sm == nullptr || sl == nullptr || !aligned16(so)))
+    return fail(LBW_ERR_INVALID, "state_o, state_m and state_l must be given together, state_o 16-byte aligned");
+  ChainPlan c;
+  int rc = make_chain_plan(p, state, &c);
+  if (rc != LBW_OK) return rc;
+  if (c.plain) return run_attention(p, false, ws, ws_bytes, stream);
+  if (p->lq == 0) return LBW_OK;
+  AttnKernelArgs& a = c.plan.a;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool ws_ok = ws != nullptr && ws_bytes >= c.plan.ws_bytes && aligned16(ws);
+  if (!ws_ok && !c.direct)
+    return fail(LBW_ERR_WORKSPACE, "workspace of %zu bytes needed (got %zu)", c.plan.ws_bytes, ws_bytes);
+  if (ws_ok && !c.plan.one_round)
+    a.queue = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(ws) + c.plan.queue_off);
+  const bool triple = p->part_o != nullptr;
+  const size_t rows = (size_t)a.B * a.H * a.Lq;
+  a.mode = kModePartials;
+  a.track_max = triple ? 1 : 0;  // the triple's m is the true row max; a normalised output needs none
+  if (!c.direct) {
+    a.part_o = static_cast<float*>(ws);
+    a.part_m = a.part_o + c.plan.splits * rows * p->head_dim;
+    a.part_l = a.part_m + c.plan.splits * rows;
+  }
+  hipError_t e = launch_attn_fwd(a, st);
+  if (e != hipSuccess) return hip_fail(e, "attention kernel launch");
+  if (c.direct) return LBW_OK;
+  MergeKernelArgs m;
+  memset(&m, 0, sizeof(m));
+  if (state) {
+    m.o[0] = so;
+    m.m[0] = sm;
+    m.l[0] = sl;
+    m.n = 1;
+  }
+  for (int s = 0; s < c.plan.splits; ++s, ++m.n) {
+    m.o[m.n] = a.part_o + s * rows * p->head_dim;
+    m.m[m.n] = a.part_m + s * rows;
+    m.l[m.n] = a.part_l + s * rows;
+  }
+  m.B = a.B; m.H = a.H; m.Lq = a.Lq; m.D = p->head_dim;
+  if (triple) {
+    m.part_o = p->part_o;
+    m.part_m = p->part_m;
+    m.part_l = p->part_l;
+  } else {
+    m.out = static_cast<uint16_t*>(p->out);
+    m.osb = p->o_stride_b; m.osl = p->o_stride_l; m.osh = p->o_stride_h;
+    m.o32 = a.o32;
+  }
+  e = launch_attn_merge(m, st);
+  if (e != hipSuccess) return hip_fail(e, "merge kernel launch");
+  return LBW_OK;
+}
+
 // ---- scratch of lbw_attention_fwd_noalloc
 // The work-queue counters and split partials of that entry point live in this file-scope device
 // array instead of a caller's workspace: each GPU the library runs on holds its own copy, at its
@@ -496,6 +596,18 @@ int lbw_attention_fwd_noalloc(const lbw_attn_params* p, void* stream) {
   void* ws = noalloc_scratch();
   if (ws == nullptr) return LBW_ERR_HIP;
   return run_attention(&q, false, ws, LBW_NOALLOC_SCRATCH_BYTES, stream);
+}
+
+size_t lbw_attention_chain_workspace_size(const lbw_attn_params* p, int32_t has_state) {
+  ChainPlan c;
+  if (make_chain_plan(p, has_state != 0, &c) != LBW_OK) return 0;
+  return c.plan.ws_bytes;
+}
+
+int lbw_attention_chain(const lbw_attn_params* p, const float* state_o, const float* state_m,
+                        const float* state_l, void* workspace, size_t workspace_bytes,
+                        void* stream) {
+  return run_chain(p, state_o, state_m, state_l, workspace, workspace_bytes, stream);
 }
 
 int lbw_attention_fwd_fp8kv(const lbw_attn_params* p, void* workspace, size_t workspace_bytes,

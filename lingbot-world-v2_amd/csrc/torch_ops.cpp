@@ -277,6 +277,82 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_partial(
   return {po, pm, pl};
 }
 
+// One call of the chain: q over the segments joined with the state (all three or none), into the
+// triple `part` (null: into p's normalised out).
+struct ChainPart {
+  at::Tensor o, m, l;
+};
+void run_chain(lbw_attn_params& p, const at::Tensor& q, const std::optional<at::Tensor>& so,
+               const std::optional<at::Tensor>& sm, const std::optional<at::Tensor>& sl,
+               ChainPart* part) {
+  const int64_t B = q.size(0), Lq = q.size(1), H = q.size(2), D = q.size(3);
+  TORCH_CHECK(so.has_value() == sm.has_value() && so.has_value() == sl.has_value(),
+              "the chain state is (O, m, l)");
+  const at::Tensor* st[3] = {so.has_value() ? &*so : nullptr, sm.has_value() ? &*sm : nullptr,
+                             sl.has_value() ? &*sl : nullptr};
+  const float* sp[3] = {nullptr, nullptr, nullptr};
+  for (int i = 0; i < 3; ++i) {
+    if (st[i] == nullptr) continue;
+    const at::Tensor& t = *st[i];
+    TORCH_CHECK(i == 0 ? t.sizes() == at::IntArrayRef({B, H, Lq, D})
+                       : t.sizes() == at::IntArrayRef({B, H, Lq}),
+                "partials differ in shape: O [B, N, Lq, D], m and l [B, N, Lq]");
+    TORCH_CHECK(t.device() == q.device(), "partials must be on one device");
+    TORCH_CHECK(t.is_contiguous() && t.scalar_type() == at::kFloat,
+                "partials must be contiguous fp32");
+    sp[i] = t.data_ptr<float>();
+  }
+  if (part != nullptr) {
+    part->o = at::empty({B, H, Lq, D}, q.options().dtype(at::kFloat));
+    part->m = at::empty({B, H, Lq}, q.options().dtype(at::kFloat));
+    part->l = at::empty({B, H, Lq}, q.options().dtype(at::kFloat));
+    p.part_o = part->o.data_ptr<float>();
+    p.part_m = part->m.data_ptr<float>();
+    p.part_l = part->l.data_ptr<float>();
+  }
+  if (Lq == 0) return;
+  run_with_workspace(
+      p, q,
+      [&](const lbw_attn_params* pp, void* ws, size_t n, void* stream) {
+        return lbw_attention_chain(pp, sp[0], sp[1], sp[2], ws, n, stream);
+      },
+      [&](const lbw_attn_params* pp) {
+        return lbw_attention_chain_workspace_size(pp, so.has_value());
+      },
+      "lbw_attention_chain");
+}
+
+std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_chain(
+    const at::Tensor& q, at::TensorList k, at::TensorList v, const std::optional<at::Tensor>& so,
+    const std::optional<at::Tensor>& sm, const std::optional<at::Tensor>& sl, int64_t kv_lo,
+    int64_t kv_hi, double softmax_scale, const std::optional<at::Tensor>& kv_lo_dev,
+    const std::optional<at::Tensor>& kv_hi_dev) {
+  c10::DeviceGuard guard(q.device());
+  lbw_attn_params p = base_params(q, k, v, kv_lo, kv_hi, softmax_scale, 0);
+  DevBounds db;
+  db.set(p, kv_lo_dev, kv_hi_dev, q);
+  ChainPart part;
+  run_chain(p, q, so, sm, sl, &part);
+  return {part.o, part.m, part.l};
+}
+
+void attention_chain_out(const at::Tensor& q, at::TensorList k, at::TensorList v,
+                         const std::optional<at::Tensor>& so, const std::optional<at::Tensor>& sm,
+                         const std::optional<at::Tensor>& sl, int64_t kv_lo, int64_t kv_hi,
+                         double softmax_scale, const at::Tensor& out,
+                         const std::optional<at::Tensor>& kv_lo_dev,
+                         const std::optional<at::Tensor>& kv_hi_dev) {
+  c10::DeviceGuard guard(q.device());
+  TORCH_CHECK(out.scalar_type() == at::kBFloat16 && out.sizes() == q.sizes() &&
+                  out.stride(3) == 1 && out.device() == q.device(),
+              "out must be bf16 [B, Lq, N, D] with a contiguous head dim");
+  lbw_attn_params p = base_params(q, k, v, kv_lo, kv_hi, softmax_scale, 0);
+  set_out(p, out, q);
+  DevBounds db;
+  db.set(p, kv_lo_dev, kv_hi_dev, q);
+  run_chain(p, q, so, sm, sl, nullptr);
+}
+
 void attention_merge_out(at::TensorList o, at::TensorList m, at::TensorList l,
                          const at::Tensor& out) {
   TORCH_CHECK(o.size() >= 1 && o.size() <= 16 && m.size() == o.size() && l.size() == o.size(),
@@ -509,6 +585,14 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_merge_partials_meta(
     at::TensorList o, at::TensorList m, at::TensorList l) {
   return {at::empty_like(o[0]), at::empty_like(m[0]), at::empty_like(l[0])};
 }
+std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_chain_meta(
+    const at::Tensor& q, at::TensorList k, at::TensorList v, const OptT&, const OptT&, const OptT&,
+    int64_t lo, int64_t hi, double scale, const OptT& dlo, const OptT& dhi) {
+  return attention_partial_meta(q, k, v, lo, hi, scale, dlo, dhi);
+}
+void attention_chain_out_meta(const at::Tensor&, at::TensorList, at::TensorList, const OptT&,
+                              const OptT&, const OptT&, int64_t, int64_t, double,
+                              const at::Tensor&, const OptT&, const OptT&) {}
 at::Tensor attention_merge_meta(at::TensorList o, at::TensorList, at::TensorList) {
   return at::empty({o[0].size(0), o[0].size(2), o[0].size(1), o[0].size(3)},
                    o[0].options().dtype(at::kBFloat16));
@@ -551,6 +635,12 @@ TORCH_LIBRARY(lbw, m) {
   m.def("attention_partial(Tensor q, Tensor[] k, Tensor[] v, int kv_lo=0, int kv_hi=-1, "
         "float softmax_scale=0., Tensor? kv_lo_dev=None, Tensor? kv_hi_dev=None) "
         "-> (Tensor, Tensor, Tensor)");
+  m.def("attention_chain(Tensor q, Tensor[] k, Tensor[] v, Tensor? state_o, Tensor? state_m, "
+        "Tensor? state_l, int kv_lo=0, int kv_hi=-1, float softmax_scale=0., "
+        "Tensor? kv_lo_dev=None, Tensor? kv_hi_dev=None) -> (Tensor, Tensor, Tensor)");
+  m.def("attention_chain_out(Tensor q, Tensor[] k, Tensor[] v, Tensor? state_o, Tensor? state_m, "
+        "Tensor? state_l, int kv_lo, int kv_hi, float softmax_scale, Tensor(a!) out, "
+        "Tensor? kv_lo_dev=None, Tensor? kv_hi_dev=None) -> ()");
   m.def("attention_merge(Tensor[] o, Tensor[] m, Tensor[] l) -> Tensor");
   m.def("attention_merge_partials(Tensor[] o, Tensor[] m, Tensor[] l) -> (Tensor, Tensor, Tensor)");
   m.def("attention_merge_out(Tensor[] o, Tensor[] m, Tensor[] l, Tensor(a!) out) -> ()");
@@ -569,6 +659,8 @@ TORCH_LIBRARY_IMPL(lbw, CUDA, m) {
   m.impl("attention_fp8kv", &attention_fp8kv);
   m.impl("attention_fp8kv_out", &attention_fp8kv_out);
   m.impl("attention_partial", &attention_partial);
+  m.impl("attention_chain", &attention_chain);
+  m.impl("attention_chain_out", &attention_chain_out);
   m.impl("attention_merge", &attention_merge);
   m.impl("attention_merge_partials", &attention_merge_partials);
   m.impl("attention_merge_out", &attention_merge_out);
@@ -584,6 +676,8 @@ TORCH_LIBRARY_IMPL(lbw, Meta, m) {
   m.impl("attention_fp8kv", &attention_fp8kv_meta);
   m.impl("attention_fp8kv_out", &attention_fp8kv_out_meta);
   m.impl("attention_partial", &attention_partial_meta);
+  m.impl("attention_chain", &attention_chain_meta);
+  m.impl("attention_chain_out", &attention_chain_out_meta);
   m.impl("attention_merge", &attention_merge_meta);
   m.impl("attention_merge_partials", &attention_merge_partials_meta);
   m.impl("attention_merge_out", &attention_merge_out_meta);

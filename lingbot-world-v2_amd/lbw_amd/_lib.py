@@ -82,7 +82,8 @@ EXPORTS = (
     "lbw_cross_attention_fwd",
     "lbw_cross_attention_dedup_fwd",
     "lbw_attention_fwd_fp8kv", "lbw_attention_fwd_noalloc", "lbw_attn_merge",
-    "lbw_attn_merge_partials", "lbw_qk_norm_rope",
+    "lbw_attn_merge_partials", "lbw_attention_chain_workspace_size", "lbw_attention_chain",
+    "lbw_qk_norm_rope",
     "lbw_kv_quant_fp8",
     "lbw_last_error", "lbw_abi_version",
 )
@@ -114,6 +115,10 @@ def _declare(lib):
     lib.lbw_attn_merge_partials.argtypes = [i32, P(vp), P(vp), P(vp), i32, i32, i32, i32, vp, vp,
                                             vp, vp]
     lib.lbw_attn_merge_partials.restype = ctypes.c_int
+    lib.lbw_attention_chain_workspace_size.argtypes = [P(AttnParams), i32]
+    lib.lbw_attention_chain_workspace_size.restype = ctypes.c_size_t
+    lib.lbw_attention_chain.argtypes = [P(AttnParams), vp, vp, vp, vp, ctypes.c_size_t, vp]
+    lib.lbw_attention_chain.restype = ctypes.c_int
     lib.lbw_qk_norm_rope.argtypes = [P(QkNormRopeParams), vp]
     lib.lbw_qk_norm_rope.restype = ctypes.c_int
     lib.lbw_kv_quant_fp8.argtypes = [vp, i32, i64, i32, i32, i64, i64, i64, vp, vp, i32, vp]

@@ -328,11 +328,10 @@ def attention_merge(parts, out: torch.Tensor | None = None) -> torch.Tensor:
     return out
 
 
-def _check_parts(parts):
-    po0 = parts[0][0]
-    B, H, Lq, D = po0.shape
+def _check_parts(parts, shape=None):
+    B, H, Lq, D = shape = parts[0][0].shape if shape is None else shape
     for o, m, l in parts:
-        if o.shape != po0.shape or m.shape != (B, H, Lq) or l.shape != (B, H, Lq):
+        if o.shape != shape or m.shape != (B, H, Lq) or l.shape != (B, H, Lq):
             raise ValueError("partials differ in shape")
         if not (o.is_contiguous() and m.is_contiguous() and l.is_contiguous()):
             raise ValueError("partials must be contiguous")
@@ -359,13 +358,27 @@ def attention_chain(q, segments, chain=None, normalize=False, *, kv_lo=None, kv_
     ``[B, Lq, N, D]``. Without it the call returns the new chain state.
 
     The state is one running triple ``(O, m, l)`` as the reference's (O, -max, sum): each call's
-    partials (attention_partial) are merged into it by ``attention_merge_partials``, so its size
+    partials are merged into it (with the pieces of the call's own keys, one launch), so its size
     does not grow with the number of calls; the normalizing call divides it out."""
     state = chain
     if segments:
-        part = attention_partial(q, segments, kv_lo=kv_lo, kv_hi=kv_hi,
-                                 softmax_scale=softmax_scale)
-        state = part if state is None else attention_merge_partials([state, part])
+        ops = _lib.ops()
+        device = q.device
+        _check_4d("q", q, device)
+        q = _as_bf16(q)
+        ks, vs = _segments(segments, device)
+        lo, hi, dlo, dhi = _bounds(kv_lo, kv_hi, device)
+        B, Lq, H, D = q.shape
+        if state is not None:
+            _check_parts([state], (B, H, Lq, D))
+        so, sm, sl = (None, None, None) if state is None else state
+        scale = 0.0 if softmax_scale is None else float(softmax_scale)
+        if not normalize:
+            return ops.attention_chain(q, ks, vs, so, sm, sl, lo, hi, scale, dlo, dhi)
+        if out is None:
+            out = torch.empty(B, Lq, H, D, dtype=torch.bfloat16, device=device)
+        ops.attention_chain_out(q, ks, vs, so, sm, sl, lo, hi, scale, out, dlo, dhi)
+        return out
     if not normalize:
         return state
     if state is None:

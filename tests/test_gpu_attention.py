@@ -447,6 +447,54 @@ def test_chain_state_is_one_running_triple(lib):
     assert float((po - ro).abs().mean() / ro.abs().mean()) <= 4e-3
 
 
+@pytest.mark.parametrize("H,Lq,lens,scale", [
+    (12, 300, [640, 641, 70], None),       # pieces of two sizes, a call too short to be cut
+    (2, 40, [1100, 0, 999], None),         # one partial q-tile per head, an empty call
+    (130, 200, [200, 300], None),          # more units than half the CUs: one piece a call
+    (300, 33, [129, 64], None),            # more units than CUs: queues
+    (3, 257, [900, 900], math.log(2.0)),   # the pre-scaled q's scale
+])
+def test_chain_calls_cut_into_pieces(lib, H, Lq, lens, scale):
+    """A chained call joins its pieces and the state in one merge: the running triple (m the true
+    row max) and the last call's output equal attention over all keys so far, into a strided out
+    as well."""
+    from lbw_amd import attention_chain
+    q, ks, vs = _case(1, Lq, H, lens, seed=H + Lq, gain=False)
+    if scale is not None:   # a q that already carries log2(e) / sqrt(d)
+        q = (q.float() * (math.log2(math.e) / math.sqrt(128))).to(torch.bfloat16)
+    qd = q.to(DEV)
+    segs = [[(k.to(DEV), v.to(DEV))] for k, v in zip(ks, vs)]
+    state = None
+    for i, s in enumerate(segs[:-1]):
+        state = attention_chain(qd, s, state, softmax_scale=scale)
+        _, (ro, rm, rl) = O.attention_ref(q, torch.cat(ks[:i + 1], 1), torch.cat(vs[:i + 1], 1),
+                                          return_partials=True, softmax_scale=scale)
+        po, pm, pl = (x.cpu() for x in state)
+        assert torch.allclose(pm, rm, rtol=1e-5, atol=1e-4)
+        assert torch.allclose(pl, rl, rtol=5e-3, atol=1e-3)
+        assert torch.allclose(po / pl[..., None], ro / rl[..., None], atol=1e-2)
+    wide = torch.zeros(1, Lq, H, 160, dtype=torch.bfloat16, device=DEV)
+    out = attention_chain(qd, segs[-1], state, normalize=True, softmax_scale=scale,
+                          out=wide[..., :128])
+    torch.cuda.synchronize()
+    assert_parity(out, O.attention_ref(q, torch.cat(ks, 1), torch.cat(vs, 1), softmax_scale=scale))
+    assert torch.all(wide[..., 128:] == 0)
+
+
+def test_chain_refuses_a_wrong_state(lib):
+    from lbw_amd import attention_chain
+    q, ks, vs = _case(1, 40, 2, [100], seed=1)
+    segs = [(ks[0].to(DEV), vs[0].to(DEV))]
+    o, m, l = attention_chain(q.to(DEV), segs)
+    for bad in ((o[:, :1].contiguous(), m, l), (o, m[..., :20].contiguous(), l),
+                (o.transpose(2, 3).contiguous().transpose(2, 3), m, l), (o.double(), m, l)):
+        with pytest.raises(ValueError):
+            attention_chain(q.to(DEV), segs, bad)
+    with pytest.raises(RuntimeError):
+        attention_chain(q.to(DEV), segs, (o, m, l), normalize=True,
+                        out=torch.empty(1, 40, 2, 128, device=DEV))
+
+
 def test_merge_partials_of_empty_rows(lib):
     """Rows with no keys in any partial (m = -inf, l = 0) merge to m = -inf, l = 0, O = 0, and
     normalise to 0, as SDPA's fully masked rows."""
