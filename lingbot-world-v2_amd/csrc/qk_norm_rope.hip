@@ -14,10 +14,10 @@
 // Two output layouts:
 // - rows: q', k' as [L, C] rows (strided), the layout the attention kernel reads;
 // - d-major: q', k' as [H, D, L] (token stride 1, a given d stride, head stride D * d stride),
-//   the layout of kernels/qk_post.py:228-306 (qk_norm_rope_t). A workgroup of 16 waves takes 16
-//   consecutive tokens, stages each 512-column slice of their outputs in LDS and writes it
-//   transposed: 32 bytes of consecutive tokens per (head, d) line. Tiles are numbered so that
-//   each XCD takes a contiguous run of them, and the two 32-byte halves of a 64-byte line are
+//   the layout of kernels/qk_post.py:228-306 (qk_norm_rope_t). A workgroup of 8 waves takes 16
+//   consecutive tokens of one tensor, stages each 512-column slice of their outputs in LDS and
+//   writes it transposed: 32 bytes of consecutive tokens per (head, d) line. Tiles are numbered so
+//   that each XCD takes a contiguous run of them, and the two 32-byte halves of a 64-byte line are
 //   usually written through the same L2.
 // With k == NULL only q is processed (kernels/qk_post.py:144-215, 308-402: x_norm_rope and
 // x_norm_rope_t3 on one tensor).
@@ -36,10 +36,12 @@ namespace lbw {
 
 constexpr int QK_WAVES = 8;                // waves per workgroup, rows layout
 constexpr int QK_MAX_BLOCKS = 512;         // rows layout: two resident per CU, looping over rows
-constexpr int QT_WAVES = 16;               // waves per workgroup, d-major layout
-constexpr int QT_ROWS = 16;                // tokens per workgroup
+constexpr int QT_ROWS = 16;                // d-major layout: tokens per workgroup
+constexpr int QT_PPC = QT_ROWS / 8;        // 16-byte pieces of a column
+constexpr int QT_TWO_PER_CU = 256;         // more (tile, tensor) items than this: two workgroups a CU
 constexpr int QT_MAX_NCH = 10;             // d-major: two rows of C <= 5120 fit 128 registers
-constexpr int QT_PITCH = 520;              // bf16 per staged token row (512 + 8: no bank clash)
+constexpr int QT_PITCH = 544;              // bf16 per staged token row: the transpose read's four
+                                           // rows of two column groups cover the 64 banks once
 constexpr int QK_MAX_TABLE = 16384;        // floats of per-axis tables held in LDS (64 KB)
 constexpr int LDS_LIMIT = 160 * 1024;
 
@@ -53,7 +55,9 @@ __host__ __device__ inline size_t qk_lds_bytes(int ntab, int C) {
 constexpr size_t QT_STAGE_BYTES = (size_t)2 * QT_ROWS * QT_PITCH * 2;
 
 size_t qk_norm_rope_lds_bytes(int ntab, int C, int layout) {
-  return qk_lds_bytes(ntab, C) + (layout == QK_LAYOUT_DMAJOR ? QT_STAGE_BYTES : 0);
+  if (layout == QK_LAYOUT_DMAJOR)
+    return (size_t)qk_table_floats(ntab) * 4 + (size_t)2 * C * 2 + QT_STAGE_BYTES;
+  return qk_lds_bytes(ntab, C);
 }
 size_t qk_norm_rope_lds_limit() { return LDS_LIMIT; }
 int qk_norm_rope_dmajor_max_dim() { return QT_MAX_NCH * 64 * 8; }
@@ -253,6 +257,13 @@ __device__ __forceinline__ void qk_copy_v(const QkNormRopeArgs& a, int row, int 
   }
 }
 
+// Four rows of one column per lane, from LDS (attn_tiles.h's transpose read).
+__device__ __forceinline__ u32x2 qk_read_tr16(int addr) {
+  typedef short shortx4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)(uintptr_t)addr));
+}
+
 // ---------------------------------------------------------------- rows layout
 // One wave per (row, tensor): with q and k the workgroup's waves pair up, wave 2j taking row
 // j's q and wave 2j + 1 its k (and half of its V copy each). A wave holds one tensor's row, so
@@ -295,105 +306,188 @@ qk_norm_rope_kernel(const QkNormRopeArgs a) {
 }
 
 // ---------------------------------------------------------------- d-major layout
-template <int NCH>
-__global__ void __launch_bounds__(QT_WAVES * 64)
+// One workgroup of W waves per (tile of QT_ROWS tokens, tensor), each wave R = QT_ROWS / W token
+// rows of it, their loads in flight while the vectors and tables fill the LDS. A 512-column slice
+// of the results is staged as rows, and each wave then writes CW columns of it: the LDS transpose read
+// (ds_read_b64_tr_b16: lane i of a 16-lane group gets four tokens of column i) gives a lane 8 or 16
+// tokens of one column, which go back to the wave's own part of the stage and out of it in the
+// order of the output, so that neighbouring lanes store neighbouring 16 bytes. The two stage
+// buffers need one barrier per slice.
+// Bound by the arithmetic (about 15 VALU operations per value, 24 us of the chip for 4680 tokens x
+// 40 heads) and the memory in turn: the two workgroups of a CU mostly load, compute and store at
+// the same time. W = 8 lets two workgroups share a CU; a workgroup alone on its CU is bound by the
+// rate at which a wave issues, and takes W = 16 (launch_nch).
+template <int NCH, int W>
+__global__ void __launch_bounds__(W * 64, 4)
 qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
+  constexpr int R = QT_ROWS / W;          // token rows per wave
+  constexpr int CW = 512 / W;             // columns of a slice that one wave writes
+  constexpr int NP = CW * QT_PPC / 64;    // pieces per lane and slice
+  constexpr int CG = CW / 16;             // 16-column groups of a wave
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  // tile numbering: XCD x (= blockIdx % 8) takes tiles [x * per, (x + 1) * per)
-  const int ntile = (a.L + QT_ROWS - 1) / QT_ROWS;
-  const int per = (ntile + 7) / 8;
-  const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if (tile >= ntile) return;  // whole workgroup, before any barrier
-
   const int C = a.C;
   const int nchunk = C / 8;
+  const int ntens = a.k != nullptr ? 2 : 1;
+  // item numbering: XCD x (= blockIdx % 8) takes items [x * per, (x + 1) * per)
+  const int nitem = (a.L + QT_ROWS - 1) / QT_ROWS * ntens;
+  const int per = (nitem + 7) / 8;
+  const int item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (item >= nitem) return;  // whole workgroup, before any barrier
+  const int t = item % ntens;
+  const int t0 = item / ntens * QT_ROWS;
+  const int nvalid = min(QT_ROWS, a.L - t0);
+
+  // LDS: [tables][bias, gamma of the tensor][2 stage buffers of QT_ROWS rows]
   float* tab = smem;
   uint16_t* vec = reinterpret_cast<uint16_t*>(smem + qk_table_floats(a.ntab));
-  uint16_t* stage = vec + 4 * C;  // [2 tensors][QT_ROWS tokens][QT_PITCH]
-  qk_fill_lds(a, tab, vec);
-  __syncthreads();
+  uint16_t* stage = vec + 2 * C;
+  constexpr int SB = QT_ROWS * QT_PITCH;  // one stage buffer
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int ntens = a.k != nullptr ? 2 : 1;
-  const int t0 = tile * QT_ROWS;
-  const int nvalid = min(QT_ROWS, a.L - t0);
-  // (token, tensor) units: with q and k, wave w takes tensor w & 1 of tokens w / 2 and
-  // w / 2 + QT_ROWS / 2; with q alone, token w. All loads are issued before any arithmetic.
-  const int t = ntens == 2 ? (wave & 1) : 0;
-  const int nunit = ntens;
-  const int tok0 = ntens == 2 ? (wave >> 1) : wave;
-  const QkTensor u = qk_tensor(a, vec, t);
-  QkOne<NCH> s[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    if (k < nunit && tok0 + (QT_ROWS / 2) * k < nvalid)
-      qk_one_load<NCH, true>(a, u, t0 + tok0 + (QT_ROWS / 2) * k, lane, s[k]);
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    if (k < nunit && tok0 + (QT_ROWS / 2) * k < nvalid)
-      qk_one_norm<NCH>(a, tab, u, t0 + tok0 + (QT_ROWS / 2) * k, lane, s[k]);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  QkTensor u = qk_tensor(a, vec, t);
+  u.bias = vec;
+  u.gamma = vec + C;
 
-  // writer role of this thread: line e of the 512-column slice, tokens [8 * half, 8 * half + 8)
-  const int e = threadIdx.x >> 1;
-  const int half = threadIdx.x & 1;
+  // vectors, then the rows, then the tables: the rows' latency covers the others'
+  constexpr int NV = (NCH + W - 1) / W;  // 16-byte chunks of a vector per thread
+  const uint16_t* src[2] = {t ? a.bk : a.bq, t ? a.wk : a.wq};
+  u32x4 xv[2][NV];
+#pragma unroll
+  for (int v = 0; v < 2; ++v)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int ch = threadIdx.x + W * 64 * i;
+      xv[v][i] = u32x4{0u, 0u, 0u, 0u};
+      if (src[v] != nullptr && ch < nchunk)
+        xv[v][i] = *reinterpret_cast<const u32x4*>(src[v] + 8 * ch);
+    }
+  QkOne<NCH> s[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    if (wave + W * k < nvalid)
+      qk_one_load<NCH, true>(a, u, t0 + wave + W * k, lane, s[k]);
+#pragma unroll
+  for (int v = 0; v < 2; ++v)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int ch = threadIdx.x + W * 64 * i;
+      if (ch < nchunk) *reinterpret_cast<u32x4*>(vec + v * C + 8 * ch) = xv[v][i];
+    }
+  const int nt2 = a.ntab / 2;  // cos/sin values come in pairs: 8-byte loads
+#pragma unroll 4
+  for (int i = threadIdx.x; i < nt2; i += W * 64)
+    reinterpret_cast<u32x2*>(tab)[i] = reinterpret_cast<const u32x2*>(a.rope)[i];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    if (wave + W * k < nvalid)
+      qk_one_norm<NCH>(a, tab, u, t0 + wave + W * k, lane, s[k]);
+
+  // the writing: per slice the wave's CW columns, as 16-byte pieces (8 tokens of a column)
+  // numbered column by column, QT_PPC to a column. A lane's transpose reads give it NP pieces of
+  // column rcol; piece id goes to chunk ((id / 4) % QT_ROWS, id % 4 + 4 (id / (4 QT_ROWS))) of the
+  // wave's part of the stage and is stored from there by lane id % 64.
+  const int i16 = lane & 15, g = lane >> 4;
+  const int rcol = 16 * (g % CG) + i16;
+  const int rtok = 8 * NP * (g / CG);
+  auto lds_at = [](const uint16_t* p) {
+    return (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint16_t*)p;
+  };
+  const int rd = lds_at(stage) + 2 * ((rtok + (i16 >> 2)) * QT_PITCH + CW * wave +
+                                      16 * (g % CG) + 4 * (i16 & 3));
+  auto piece_at = [&](int id) {  // element offset in a stage buffer
+    return (id / 4 % QT_ROWS) * QT_PITCH + CW * wave + 8 * (id % 4 + 4 * (id / (4 * QT_ROWS)));
+  };
+  uint16_t* const out = t ? a.ko : a.qo;
+  const int64_t os = t ? a.kos : a.qos;
+  const int ntok = nvalid - 8 * (lane % QT_PPC);  // tokens of this lane's pieces that exist (>= 8: all)
+  const int64_t lane_out = (int64_t)(lane / QT_PPC) * os + 8 * (lane % QT_PPC);
+  const bool vec_ok = (t ? a.ko_vec : a.qo_vec) != 0;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
+    uint16_t* sb = stage + (i & 1) * SB;
     const int ch = lane + 64 * i;
     if (i + 1 < NCH || ch < nchunk) {
+      const u32x4 bv = *reinterpret_cast<const u32x4*>(u.bias + 8 * ch);
+      const u32x4 gv = *reinterpret_cast<const u32x4*>(u.gamma + 8 * ch);
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int tok = tok0 + (QT_ROWS / 2) * k;
-        if (k < nunit && tok < nvalid)
-          *reinterpret_cast<u32x4*>(stage + (t * QT_ROWS + tok) * QT_PITCH + 8 * lane) =
-              qk_finish(s[k].x[i], *reinterpret_cast<const u32x4*>(u.bias + 8 * ch),
-                        *reinterpret_cast<const u32x4*>(u.gamma + 8 * ch), s[k].r, s[k].c,
-                        s[k].sn, s[k].rotate, u.scale);
-      }
+      for (int k = 0; k < R; ++k)
+        if (wave + W * k < nvalid)
+          *reinterpret_cast<u32x4*>(sb + (wave + W * k) * QT_PITCH + 8 * lane) =
+              qk_finish(s[k].x[i], bv, gv, s[k].r, s[k].c, s[k].sn, s[k].rotate, u.scale);
     }
     __syncthreads();
-    // line e = head * D + d of the slice starts at col * d_stride
-    const int col = 512 * i + e;
-    if (col < C) {
-      for (int tw = 0; tw < ntens; ++tw) {
-        const uint16_t* sp = stage + (tw * QT_ROWS + 8 * half) * QT_PITCH + e;
-        uint16_t v[8];
+    const int col0 = 512 * i + CW * wave;  // column e = head * D + d starts at e * d_stride
+    if (col0 >= C) continue;
+    u32x2 x[2 * NP];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = sp[j * QT_PITCH];
-        uint16_t* dst = (tw ? a.ko : a.qo) + (int64_t)col * (tw ? a.kos : a.qos) + t0 + 8 * half;
-        const bool vec_ok = tw ? a.ko_vec : a.qo_vec;
-        if (vec_ok && 8 * half + 8 <= nvalid) {
-          u32x4 w;
+    for (int j = 0; j < 2 * NP; ++j)
+      x[j] = qk_read_tr16(rd + 2 * ((i & 1) * SB + 4 * j * QT_PITCH));
 #pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = (uint32_t)v[2 * j] | ((uint32_t)v[2 * j + 1] << 16);
-          *reinterpret_cast<u32x4*>(dst) = w;
+    for (int j = 0; j < NP; ++j)
+      *reinterpret_cast<u32x4*>(sb + piece_at(rcol * QT_PPC + rtok / 8 + j)) =
+          u32x4{x[2 * j][0], x[2 * j][1], x[2 * j + 1][0], x[2 * j + 1][1]};
+    if (vec_ok) {
+#pragma unroll
+      for (int j = 0; j < NP; ++j) {
+        const int cj = col0 + 64 / QT_PPC * j;  // (wave-uniform) column of lane 0
+        const u32x4 v = *reinterpret_cast<const u32x4*>(sb + piece_at(64 * j + lane));
+        if (cj + lane / QT_PPC >= C) continue;
+        uint16_t* dst = out + cj * os + t0 + lane_out;
+        if (ntok >= 8) {
+          *reinterpret_cast<u32x4*>(dst) = v;
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (8 * half + j < nvalid) dst[j] = v[j];
+          for (int e = 0; e < 7; ++e)
+            if (e < ntok) dst[e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
         }
       }
+    } else {
+      // outputs that 16-byte stores cannot reach: consecutive lanes take consecutive tokens of a column
+      for (int e = lane; e < CW * QT_ROWS; e += 64) {
+        const int col = e / QT_ROWS, tok = e % QT_ROWS;
+        const uint16_t v = sb[piece_at(col * QT_PPC + tok / 8) + tok % 8];
+        if (col0 + col < C && tok < nvalid) out[(int64_t)(col0 + col) * os + t0 + tok] = v;
+      }
     }
-    __syncthreads();  // the slice is read before the next one is staged
   }
-  if (a.v != nullptr && wave < nvalid) qk_copy_v<NCH, true>(a, t0 + wave, lane, 0, 1);
+  if (a.v != nullptr) {
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (wave + W * k < nvalid)
+        qk_copy_v<NCH, true>(a, t0 + wave + W * k, lane, t, ntens);
+  }
+}
+
+template <int NCH, int W>
+static hipError_t launch_dmajor(const QkNormRopeArgs& a, int items, hipStream_t stream) {
+  static hipError_t attr = hipFuncSetAttribute(
+      (const void*)qk_norm_rope_dmajor_kernel<NCH, W>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      (int)(qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR) < LDS_LIMIT
+                ? qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR)
+                : LDS_LIMIT));
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((qk_norm_rope_dmajor_kernel<NCH, W>), dim3(8 * ((items + 7) / 8)), dim3(W * 64),
+                     qk_norm_rope_lds_bytes(a.ntab, a.C, QK_LAYOUT_DMAJOR), stream, a);
+  return hipGetLastError();
 }
 
 template <int NCH>
 static hipError_t launch_nch(const QkNormRopeArgs& a, hipStream_t stream) {
   if (a.layout == QK_LAYOUT_DMAJOR) {
-    if constexpr (NCH > QT_MAX_NCH) return hipErrorInvalidValue;  // rejected by the host check
-    static hipError_t attr = hipFuncSetAttribute(
-        (const void*)qk_norm_rope_dmajor_kernel<NCH>, hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)(qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR) < LDS_LIMIT
-                  ? qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR)
-                  : LDS_LIMIT));
-    if (attr != hipSuccess) return attr;
-    const int ntile = (a.L + QT_ROWS - 1) / QT_ROWS;
-    const int blocks = 8 * ((ntile + 7) / 8);
-    hipLaunchKernelGGL(qk_norm_rope_dmajor_kernel<NCH>, dim3(blocks), dim3(QT_WAVES * 64),
-                       qk_norm_rope_lds_bytes(a.ntab, a.C, QK_LAYOUT_DMAJOR), stream, a);
-    return hipGetLastError();
+    if constexpr (NCH > QT_MAX_NCH) {
+      return hipErrorInvalidValue;  // rejected by the host check
+    } else {
+    // (tile, tensor) items that leave a CU one workgroup take 16 waves of one row, more take 8 of
+    // two. Kernel times at 40 heads, us, W = 8 and W = 16 (and the form before both, one workgroup of
+    // 16 waves per tile of both tensors that read the stage by elements): 2048 tokens, 256 items,
+    // 25.6, 23.1 (37.4); 2560, 320 items, 34.0, 38.5 (38.9); 3600 35.3, 42.0 (39.7); 4680 57.8, 57.4
+    // (70.5); 9360 101.5, 98.2 (106.4)
+    const int items = (a.L + QT_ROWS - 1) / QT_ROWS * (a.k != nullptr ? 2 : 1);
+    return items > QT_TWO_PER_CU ? launch_dmajor<NCH, 8>(a, items, stream)
+                                 : launch_dmajor<NCH, 16>(a, items, stream);
+    }
   }
   static hipError_t attr = hipFuncSetAttribute((const void*)qk_norm_rope_kernel<NCH>,
                                                hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -151,6 +151,36 @@ def test_qk_norm_rope_t_into_cache_slot(lib, offset):
     assert torch.all(v_out[:offset] == 0) and torch.all(v_out[offset + L:] == 0)
 
 
+@pytest.mark.parametrize("L", [1, 16, 17, 31, 41])
+@pytest.mark.parametrize("C", [128, 640, 5120])
+@pytest.mark.parametrize("cap", [48, 45])
+def test_dmajor_tiles_equal_rows(lib, L, C, cap):
+    """The d-major kernel at the edges of its 16-token tiles and 512-column slices, with aligned
+    and odd d strides: the same arithmetic as the rows layout, so bit for bit its values; the
+    tokens around the slot and the copied V stay right. One tensor (k = None) as well."""
+    from lbw_amd import causal_rope_tables, qk_norm_rope_, wan_rope_freqs
+    H, D = C // 128, 128
+    grid = (1, 3, 10)              # tokens from 30 on are not rotated
+    q, k, bq, bk, wq, wk = _dev(*_inputs(L, C, seed=L + C))
+    v = torch.randn(L, C, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    tabs = causal_rope_tables(wan_rope_freqs(128), grid, 2, device=DEV)
+    print(f"case L={L} C={C} cap={cap}", flush=True)
+    rq, rk = torch.empty_like(q), torch.empty_like(k)
+    qk_norm_rope_(q, k, bq, bk, wq, wk, tabs, 1e-6, H, q_out=rq, k_out=rk, q_scale=0.5)
+    for kk in (k, None):
+        cq = torch.zeros(H, D, cap, dtype=torch.bfloat16, device=DEV)
+        ck, v_out = torch.zeros_like(cq), torch.zeros_like(v)
+        qk_norm_rope_(q, kk, bq, None if kk is None else bk, wq, None if kk is None else wk, tabs,
+                      1e-6, H, q_out=cq[:, :, :L], k_out=None if kk is None else ck[:, :, :L],
+                      q_scale=0.5, layout="dmajor", v=v, v_out=v_out)
+        torch.cuda.synchronize()
+        assert torch.equal(_rows_of(cq[:, :, :L]), rq)
+        if kk is not None:
+            assert torch.equal(_rows_of(ck[:, :, :L]), rk)
+        assert torch.all(cq[:, :, L:] == 0) and torch.all(ck[:, :, L:] == 0)
+        assert torch.equal(v_out, v)
+
+
 def test_single_tensor_and_fused_projection_forms(lib):
     """x_norm_rope (rows), x_norm_rope_t3 / qk_norm_rope3 / qk_norm_rope_t3 on the fused
     projection [L, 3C] (kernels/qk_post.py:81-86, 166-215, 221-225, 331-402), and the rows
