@@ -280,7 +280,8 @@ qk_norm_rope_kernel(const QkNormRopeArgs a) {
   __syncthreads();
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  // (a scalar, so that the row's position, branches and addresses are; 114 registers before, 96)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ntens = a.k != nullptr ? 2 : 1;
   const int t = wave % ntens;
   const int rows_per_block = QK_WAVES / ntens;
