@@ -64,6 +64,16 @@ __device__ __forceinline__ void barrier_nofence() {
   asm volatile("" ::: "memory");
 }
 
+// Orders one wave's LDS accesses before and after it across lanes: data that some lanes of the
+// wave wrote and others read (or read and others overwrite) with no workgroup barrier between.
+// The hardware runs a wave's LDS instructions in order; this keeps the compiler, which sees one
+// lane's addresses only, from exchanging them. No instruction of its own.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ float wave_reduce_sum(float v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);

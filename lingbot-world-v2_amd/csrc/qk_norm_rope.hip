@@ -425,10 +425,12 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
 #pragma unroll
     for (int j = 0; j < 2 * NP; ++j)
       x[j] = qk_read_tr16(rd + 2 * ((i & 1) * SB + 4 * j * QT_PITCH));
+    wave_lds_fence();
 #pragma unroll
     for (int j = 0; j < NP; ++j)
       *reinterpret_cast<u32x4*>(sb + piece_at(rcol * QT_PPC + rtok / 8 + j)) =
           u32x4{x[2 * j][0], x[2 * j][1], x[2 * j + 1][0], x[2 * j + 1][1]};
+    wave_lds_fence();
     if (vec_ok) {
 #pragma unroll
       for (int j = 0; j < NP; ++j) {

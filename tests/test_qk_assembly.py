@@ -1,0 +1,64 @@
+"""What the gfx950 assembly of the q/k kernels (csrc/qk_norm_rope.hip) must show, since no run
+shows it reliably: in the d-major kernel the lanes of a wave exchange values through LDS with no
+workgroup barrier between, so the compiler may not move the LDS accesses past one another there."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "lingbot-world-v2_amd", "csrc")
+ASM = os.path.join(HERE, "..", "_build", "csrc", "qk_norm_rope.s")
+
+pytestmark = pytest.mark.skipif(not shutil.which("hipcc") and not os.path.exists("/opt/rocm/bin/hipcc"),
+                                reason="no hipcc")
+
+
+@pytest.fixture(scope="module")
+def asm():
+    subprocess.run(["make", "-C", CSRC, "../../_build/csrc/qk_norm_rope.s"], check=True,
+                   capture_output=True)
+    return open(ASM).read()
+
+
+def _dmajor_kernels(asm):
+    """{(chunks, waves): lines} of the d-major kernel's instances."""
+    out = {}
+    for m in re.finditer(r"^_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)E\S*:.*?^\.Lfunc_end",
+                         asm, re.M | re.S):
+        out[int(m.group(1)), int(m.group(2))] = m.group(0).splitlines()
+    return out
+
+
+def unfenced(lines):
+    """Line numbers of the LDS accesses of the exchange (transpose reads, stores over what they
+    read, reads of what other lanes stored) with no wave barrier before them."""
+    bad, state = [], None
+    for n, line in enumerate(lines):
+        op = line.split()[0] if line.split() else ""
+        if "; wave barrier" in line:
+            state = {"reads": "stores next", "stores": None}.get(state, state)
+        elif op.startswith("ds_read_b64_tr"):
+            state = "reads"
+        elif op.startswith("ds_write") and state in ("reads", "stores next"):
+            if state == "reads":
+                bad.append(n)
+            state = "stores"
+        elif op.startswith("ds_read") and state in ("reads", "stores"):
+            if state == "stores":
+                bad.append(n)
+                state = None
+    return bad
+
+
+def test_lane_exchanges_are_fenced(asm):
+    kernels = _dmajor_kernels(asm)
+    assert len(kernels) == 20  # 1..10 chunks per lane, 8 and 16 waves
+    for inst, lines in kernels.items():
+        assert any("ds_read_b64_tr" in l for l in lines), inst
+        assert not unfenced(lines), inst
+    # the check sees a missing fence: the same listing without either
+    lines = [l for l in kernels[4, 8] if "; wave barrier" not in l]
+    assert unfenced(lines)
