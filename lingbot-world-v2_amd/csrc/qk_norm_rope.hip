@@ -233,9 +233,8 @@ __device__ __forceinline__ u32x4 qk_finish(const u32x4& x, const u32x4& bv, cons
   return ov;
 }
 
-// copy the chunks i of a V row with i % nsplit == part (the row's waves share the copy); NT:
-// as for qk_load16, the stores too
-template <int NCH, bool NT>
+// copy the chunks i of a V row with i % nsplit == part (the row's waves share the copy)
+template <int NCH>
 __device__ __forceinline__ void qk_copy_v(const QkNormRopeArgs& a, int row, int lane, int part,
                                           int nsplit) {
   const int nchunk = a.C / 8;
@@ -246,14 +245,39 @@ __device__ __forceinline__ void qk_copy_v(const QkNormRopeArgs& a, int row, int 
   for (int i = 0; i < NCH; ++i) {
     const int ch = lane + 64 * i;
     if (i % nsplit == part && (i + 1 < NCH || ch < nchunk))
-      xv[i] = qk_load16<NT>(vs + 8 * ch);
+      xv[i] = *reinterpret_cast<const u32x4*>(vs + 8 * ch);
   }
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int ch = lane + 64 * i;
     if (i % nsplit == part && (i + 1 < NCH || ch < nchunk))
-      if constexpr (NT) __builtin_nontemporal_store(xv[i], reinterpret_cast<u32x4*>(vd + 8 * ch));
-      else *reinterpret_cast<u32x4*>(vd + 8 * ch) = xv[i];
+      *reinterpret_cast<u32x4*>(vd + 8 * ch) = xv[i];
+  }
+}
+
+// the same for the d-major kernel, with the number of parts known to the compiler and the
+// non-temporal hint on both sides (qk_load16). The form above takes more registers than that kernel
+// has: the chunks of a row of up to 8 become one array of 32 registers that is merged whole at
+// every chunk's branch. It spilled 132 to 772 bytes per lane at 6 to 8 chunks, and with the V copy
+// 3600 tokens x 32 heads took 324 us where this form takes 46.
+template <int NCH, int NSPLIT>
+__device__ __forceinline__ void qk_copy_v_part(const QkNormRopeArgs& a, int row, int lane,
+                                               int part) {
+  constexpr int N = (NCH + NSPLIT - 1) / NSPLIT;
+  const int nchunk = a.C / 8;
+  const uint16_t* vs = a.v + a.vs * row;
+  uint16_t* vd = a.vo + a.vos * row;
+  u32x4 xv[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int ch = lane + 64 * (NSPLIT * j + part);
+    if (NSPLIT * (j + 1) < NCH || ch < nchunk) xv[j] = qk_load16<true>(vs + 8 * ch);
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int ch = lane + 64 * (NSPLIT * j + part);
+    if (NSPLIT * (j + 1) < NCH || ch < nchunk)
+      __builtin_nontemporal_store(xv[j], reinterpret_cast<u32x4*>(vd + 8 * ch));
   }
 }
 
@@ -302,7 +326,7 @@ qk_norm_rope_kernel(const QkNormRopeArgs a) {
                       *reinterpret_cast<const u32x4*>(u.gamma + 8 * ch), s.r, s.c, s.sn,
                       s.rotate, u.scale);
     }
-    if (a.v != nullptr) qk_copy_v<NCH, false>(a, row, lane, t, ntens);
+    if (a.v != nullptr) qk_copy_v<NCH>(a, row, lane, t, ntens);
   }
 }
 
@@ -410,13 +434,22 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
     uint16_t* sb = stage + (i & 1) * SB;
     const int ch = lane + 64 * i;
     if (i + 1 < NCH || ch < nchunk) {
-      const u32x4 bv = *reinterpret_cast<const u32x4*>(u.bias + 8 * ch);
-      const u32x4 gv = *reinterpret_cast<const u32x4*>(u.gamma + 8 * ch);
+      const u32x4* const bp = reinterpret_cast<const u32x4*>(u.bias + 8 * ch);
+      const u32x4* const gp = reinterpret_cast<const u32x4*>(u.gamma + 8 * ch);
+      u32x4 bv = *bp, gv = *gp;
 #pragma unroll
-      for (int k = 0; k < R; ++k)
+      for (int k = 0; k < R; ++k) {
+        // two rows of more than 8 chunks leave no registers to keep the vectors for the second:
+        // read again (36 to 44 bytes of scratch per lane else)
+        if (NCH > 8 && k > 0) {
+          asm volatile("" ::: "memory");
+          bv = *bp;
+          gv = *gp;
+        }
         if (wave + W * k < nvalid)
           *reinterpret_cast<u32x4*>(sb + (wave + W * k) * QT_PITCH + 8 * lane) =
               qk_finish(s[k].x[i], bv, gv, s[k].r, s[k].c, s[k].sn, s[k].rotate, u.scale);
+      }
     }
     __syncthreads();
     const int col0 = 512 * i + CW * wave;  // column e = head * D + d starts at e * d_stride
@@ -458,8 +491,10 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
   if (a.v != nullptr) {
 #pragma unroll
     for (int k = 0; k < R; ++k)
-      if (wave + W * k < nvalid)
-        qk_copy_v<NCH, true>(a, t0 + wave + W * k, lane, t, ntens);
+      if (wave + W * k < nvalid) {
+        if (ntens == 2) qk_copy_v_part<NCH, 2>(a, t0 + wave + W * k, lane, t);
+        else qk_copy_v_part<NCH, 1>(a, t0 + wave + W * k, lane, 0);
+      }
   }
 }
 

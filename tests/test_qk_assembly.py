@@ -1,6 +1,7 @@
 """What the gfx950 assembly of the q/k kernels (csrc/qk_norm_rope.hip) must show, since no run
 shows it reliably: in the d-major kernel the lanes of a wave exchange values through LDS with no
-workgroup barrier between, so the compiler may not move the LDS accesses past one another there."""
+workgroup barrier between, so the compiler may not move the LDS accesses past one another there; and
+none of that kernel's instances, which hold whole rows under a limit of 128 registers, spills."""
 import os
 import re
 import shutil
@@ -62,3 +63,15 @@ def test_lane_exchanges_are_fenced(asm):
     # the check sees a missing fence: the same listing without either
     lines = [l for l in kernels[4, 8] if "; wave barrier" not in l]
     assert unfenced(lines)
+
+
+def test_dmajor_kernels_use_no_scratch(asm):
+    spilled = {}
+    for block in re.split(r"^  - \.", asm, flags=re.M):
+        m = re.search(r"\.name: +_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)E", block)
+        if m:
+            spilled[int(m.group(1)), int(m.group(2))] = tuple(
+                int(re.search(rf"\.{key}: +(\d+)", block).group(1))
+                for key in ("private_segment_fixed_size", "vgpr_spill_count", "sgpr_spill_count"))
+    assert len(spilled) == 20
+    assert all(v == (0, 0, 0) for v in spilled.values()), spilled
