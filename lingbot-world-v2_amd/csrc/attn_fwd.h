@@ -106,7 +106,7 @@ struct QkNormRopeArgs {
 };
 constexpr int QK_LAYOUT_ROWS = 0;
 constexpr int QK_LAYOUT_DMAJOR = 1;
-hipError_t launch_qk_norm_rope(const QkNormRopeArgs& a, hipStream_t stream);
+hipError_t launch_qk_norm_rope(const QkNormRopeArgs& a, int num_cus, hipStream_t stream);
 int qk_norm_rope_max_table_floats();
 size_t qk_norm_rope_lds_bytes(int ntab, int C, int layout);
 size_t qk_norm_rope_lds_limit();

@@ -755,7 +755,7 @@ int lbw_qk_norm_rope(const lbw_qk_norm_rope_params* p, void* stream) {
   a.q_scale = p->q_out_scale; a.k_scale = p->k_out_scale;
   a.v = static_cast<const uint16_t*>(p->v); a.vs = p->v_stride;
   a.vo = static_cast<uint16_t*>(p->v_out); a.vos = p->v_out_stride;
-  hipError_t e = launch_qk_norm_rope(a, static_cast<hipStream_t>(stream));
+  hipError_t e = launch_qk_norm_rope(a, num_cus(), static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "qk_norm_rope launch");
   return LBW_OK;
 }

@@ -14,7 +14,7 @@
 // Two output layouts:
 // - rows: q', k' as [L, C] rows (strided), the layout the attention kernel reads;
 // - d-major: q', k' as [H, D, L] (token stride 1, a given d stride, head stride D * d stride),
-//   the layout of kernels/qk_post.py:228-306 (qk_norm_rope_t). A workgroup of 8 waves takes 16
+//   the layout of kernels/qk_post.py:228-306 (qk_norm_rope_t). A workgroup of 8 or 16 waves takes 16
 //   consecutive tokens of one tensor, stages each 512-column slice of their outputs in LDS and
 //   writes it transposed: 32 bytes of consecutive tokens per (head, d) line. Tiles are numbered so
 //   that each XCD takes a contiguous run of them, and the two 32-byte halves of a 64-byte line are
@@ -38,7 +38,6 @@ constexpr int QK_WAVES = 8;                // waves per workgroup, rows layout
 constexpr int QK_MAX_BLOCKS = 512;         // rows layout: two resident per CU, looping over rows
 constexpr int QT_ROWS = 16;                // d-major layout: tokens per workgroup
 constexpr int QT_PPC = QT_ROWS / 8;        // 16-byte pieces of a column
-constexpr int QT_TWO_PER_CU = 256;         // more (tile, tensor) items than this: two workgroups a CU
 constexpr int QT_MAX_NCH = 10;             // d-major: two rows of C <= 5120 fit 128 registers
 constexpr int QT_PITCH = 544;              // bf16 per staged token row: the transpose read's four
                                            // rows of two column groups cover the 64 banks once
@@ -512,19 +511,27 @@ static hipError_t launch_dmajor(const QkNormRopeArgs& a, int items, hipStream_t 
 }
 
 template <int NCH>
-static hipError_t launch_nch(const QkNormRopeArgs& a, hipStream_t stream) {
+static hipError_t launch_nch(const QkNormRopeArgs& a, int num_cus, hipStream_t stream) {
   if (a.layout == QK_LAYOUT_DMAJOR) {
     if constexpr (NCH > QT_MAX_NCH) {
       return hipErrorInvalidValue;  // rejected by the host check
     } else {
-    // (tile, tensor) items that leave a CU one workgroup take 16 waves of one row, more take 8 of
-    // two. Kernel times at 40 heads, us, W = 8 and W = 16 (and the form before both, one workgroup of
-    // 16 waves per tile of both tensors that read the stage by elements): 2048 tokens, 256 items,
-    // 25.6, 23.1 (37.4); 2560, 320 items, 34.0, 38.5 (38.9); 3600 35.3, 42.0 (39.7); 4680 57.8, 57.4
-    // (70.5); 9360 101.5, 98.2 (106.4)
-    const int items = (a.L + QT_ROWS - 1) / QT_ROWS * (a.k != nullptr ? 2 : 1);
-    return items > QT_TWO_PER_CU ? launch_dmajor<NCH, 8>(a, items, stream)
-                                 : launch_dmajor<NCH, 16>(a, items, stream);
+      // 16 waves of one row or 8 of two. Kernel times, us, W = 8 and W = 16, inputs from HBM:
+      // - one workgroup per CU (items or LDS leave no second): 16, a lone one is bound by the rate
+      //   at which its waves issue. 1560 tokens x 40 heads, 196 items, 25.9, 23.5.
+      // - 3 to 5 chunks: 16, whose 64 registers let two share a CU as well. 3600 x 20 heads 24.4,
+      //   23.1; 9360 64.4, 56.5; 4680 x 12 26.9, 25.6 (2 chunks, 4680 x 5: 15.6, 16.3).
+      // - above, up to two items per CU: 8, two workgroups side by side where 16 take two rounds.
+      //   2560 x 40, 320 items, 34.6, 39.1; 3600, 450, 41.5, 45.8; 3600 x 24 26.8, 32.3.
+      // - more items: 8 up to 8 chunks (10800 x 24 85, 92; x 32 108, 110), 16 for longer rows
+      //   (4680 x 40 72.2, 64.6; 9360 119, 110; 10800 143, 128).
+      const int items = (a.L + QT_ROWS - 1) / QT_ROWS * (a.k != nullptr ? 2 : 1);
+      const bool pair = 2 * qk_norm_rope_lds_bytes(a.ntab, a.C, QK_LAYOUT_DMAJOR) <= LDS_LIMIT;
+      if constexpr (NCH < 3 || NCH > 5) {
+        if (items > num_cus && pair && (NCH < 9 || items <= 2 * num_cus))
+          return launch_dmajor<NCH, 8>(a, items, stream);
+      }
+      return launch_dmajor<NCH, 16>(a, items, stream);
     }
   }
   static hipError_t attr = hipFuncSetAttribute((const void*)qk_norm_rope_kernel<NCH>,
@@ -542,25 +549,25 @@ static hipError_t launch_nch(const QkNormRopeArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_qk_norm_rope(const QkNormRopeArgs& a, hipStream_t stream) {
+hipError_t launch_qk_norm_rope(const QkNormRopeArgs& a, int num_cus, hipStream_t stream) {
   const int nch = (a.C / 8 + 63) / 64;
   switch (nch) {
-    case 1: return launch_nch<1>(a, stream);
-    case 2: return launch_nch<2>(a, stream);
-    case 3: return launch_nch<3>(a, stream);
-    case 4: return launch_nch<4>(a, stream);
-    case 5: return launch_nch<5>(a, stream);
-    case 6: return launch_nch<6>(a, stream);
-    case 7: return launch_nch<7>(a, stream);
-    case 8: return launch_nch<8>(a, stream);
-    case 9: return launch_nch<9>(a, stream);
-    case 10: return launch_nch<10>(a, stream);
-    case 11: return launch_nch<11>(a, stream);
-    case 12: return launch_nch<12>(a, stream);
-    case 13: return launch_nch<13>(a, stream);
-    case 14: return launch_nch<14>(a, stream);
-    case 15: return launch_nch<15>(a, stream);
-    case 16: return launch_nch<16>(a, stream);
+    case 1: return launch_nch<1>(a, num_cus, stream);
+    case 2: return launch_nch<2>(a, num_cus, stream);
+    case 3: return launch_nch<3>(a, num_cus, stream);
+    case 4: return launch_nch<4>(a, num_cus, stream);
+    case 5: return launch_nch<5>(a, num_cus, stream);
+    case 6: return launch_nch<6>(a, num_cus, stream);
+    case 7: return launch_nch<7>(a, num_cus, stream);
+    case 8: return launch_nch<8>(a, num_cus, stream);
+    case 9: return launch_nch<9>(a, num_cus, stream);
+    case 10: return launch_nch<10>(a, num_cus, stream);
+    case 11: return launch_nch<11>(a, num_cus, stream);
+    case 12: return launch_nch<12>(a, num_cus, stream);
+    case 13: return launch_nch<13>(a, num_cus, stream);
+    case 14: return launch_nch<14>(a, num_cus, stream);
+    case 15: return launch_nch<15>(a, num_cus, stream);
+    case 16: return launch_nch<16>(a, num_cus, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -181,6 +181,39 @@ def test_dmajor_tiles_equal_rows(lib, L, C, cap):
         assert torch.equal(v_out, v)
 
 
+@pytest.mark.parametrize("C,L", [(256, 2061), (640, 2061), (1024, 4173), (3072, 2061), (3072, 4173),
+                                 (3584, 2173), (4096, 2061), (4224, 2061), (4608, 4173),
+                                 (5120, 2061), (5120, 4173)])
+@pytest.mark.parametrize("pad", [3, 6])
+def test_dmajor_many_tiles_equal_rows(lib, C, L, pad):
+    """More (16-token tile, tensor) items than CUs, up to two per CU and beyond, with a partial last
+    tile: rows of every length class, two per wave and one, aligned and odd d strides, with the V
+    copy, both tensors and one (4173 tokens: above the CUs with one tensor as well)."""
+    from lbw_amd import causal_rope_tables, qk_norm_rope_, wan_rope_freqs
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 2 * ((L + 15) // 16) > cus and (L < 4000 or (L + 15) // 16 > cus)
+    H, D = C // 128, 128
+    cap = L + pad                  # the d stride: L + 3 is a multiple of 8, L + 6 odd
+    q, k, bq, bk, wq, wk = _dev(*_inputs(L, C, seed=L + C))
+    v = torch.randn(L, C, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    tabs = causal_rope_tables(wan_rope_freqs(128), (2, 20, 51), 2, device=DEV)   # 2040 rotated
+    print(f"case L={L} C={C} cap={cap}", flush=True)
+    rq, rk = torch.empty_like(q), torch.empty_like(k)
+    qk_norm_rope_(q, k, bq, bk, wq, wk, tabs, 1e-6, H, q_out=rq, k_out=rk, q_scale=0.5)
+    for kk in (k, None):
+        cq = torch.zeros(H, D, cap, dtype=torch.bfloat16, device=DEV)
+        ck, v_out = torch.zeros_like(cq), torch.zeros_like(v)
+        qk_norm_rope_(q, kk, bq, None if kk is None else bk, wq, None if kk is None else wk, tabs,
+                      1e-6, H, q_out=cq[:, :, :L], k_out=None if kk is None else ck[:, :, :L],
+                      q_scale=0.5, layout="dmajor", v=v, v_out=v_out)
+        torch.cuda.synchronize()
+        assert torch.equal(_rows_of(cq[:, :, :L]), rq)
+        if kk is not None:
+            assert torch.equal(_rows_of(ck[:, :, :L]), rk)
+        assert torch.all(cq[:, :, L:] == 0) and torch.all(ck[:, :, L:] == 0)
+        assert torch.equal(v_out, v)
+
+
 def test_single_tensor_and_fused_projection_forms(lib):
     """x_norm_rope (rows), x_norm_rope_t3 / qk_norm_rope3 / qk_norm_rope_t3 on the fused
     projection [L, 3C] (kernels/qk_post.py:81-86, 166-215, 221-225, 331-402), and the rows
