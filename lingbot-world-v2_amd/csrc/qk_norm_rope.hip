@@ -15,8 +15,8 @@
 // - rows: q', k' as [L, C] rows (strided), the layout the attention kernel reads;
 // - d-major: q', k' as [H, D, L] (token stride 1, a given d stride, head stride D * d stride),
 //   the layout of kernels/qk_post.py:228-306 (qk_norm_rope_t). A workgroup of 8 or 16 waves takes 16
-//   consecutive tokens of one tensor, stages each 512-column slice of their outputs in LDS and
-//   writes it transposed: 32 bytes of consecutive tokens per (head, d) line. Tiles are numbered so
+//   or 32 consecutive tokens of one tensor, stages each 512-column slice of their outputs in LDS
+//   and writes it transposed: 32 or 64 bytes of consecutive tokens per (head, d) line. Tiles are numbered so
 //   that each XCD takes a contiguous run of them, and the two 32-byte halves of a 64-byte line are
 //   usually written through the same L2.
 // With k == NULL only q is processed (kernels/qk_post.py:144-215, 308-402: x_norm_rope and
@@ -36,13 +36,14 @@ namespace lbw {
 
 constexpr int QK_WAVES = 8;                // waves per workgroup, rows layout
 constexpr int QK_MAX_BLOCKS = 512;         // rows layout: two resident per CU, looping over rows
-constexpr int QT_ROWS = 16;                // d-major layout: tokens per workgroup
-constexpr int QT_PPC = QT_ROWS / 8;        // 16-byte pieces of a column
+constexpr int QT_TILE = 16, QT_LONG = 32;  // d-major layout: tokens per workgroup, long chunks
 constexpr int QT_MAX_NCH = 10;             // d-major: two rows of C <= 5120 fit 128 registers
 constexpr int QT_PITCH = 544;              // bf16 per staged token row: the transpose read's four
                                            // rows of two column groups cover the 64 banks once
 constexpr int QK_MAX_TABLE = 16384;        // floats of per-axis tables held in LDS (64 KB)
 constexpr int LDS_LIMIT = 160 * 1024;
+static_assert(QK_MAX_TABLE * 4 + 2 * QT_MAX_NCH * 512 * 2 + 2 * QT_LONG * QT_PITCH * 2 <= LDS_LIMIT,
+              "the larger tile fits beside any tables");
 
 int qk_norm_rope_max_table_floats() { return QK_MAX_TABLE; }
 
@@ -51,12 +52,13 @@ __host__ __device__ inline int qk_table_floats(int ntab) { return (ntab + 3) & ~
 __host__ __device__ inline size_t qk_lds_bytes(int ntab, int C) {
   return (size_t)qk_table_floats(ntab) * 4 + (size_t)4 * C * 2;
 }
-constexpr size_t QT_STAGE_BYTES = (size_t)2 * QT_ROWS * QT_PITCH * 2;
+// d-major: [tables][bias, gamma][2 stage buffers of a tile's rows]
+static size_t qt_lds_bytes(int ntab, int C, int tile) {
+  return (size_t)qk_table_floats(ntab) * 4 + (size_t)2 * C * 2 + (size_t)2 * tile * QT_PITCH * 2;
+}
 
 size_t qk_norm_rope_lds_bytes(int ntab, int C, int layout) {
-  if (layout == QK_LAYOUT_DMAJOR)
-    return (size_t)qk_table_floats(ntab) * 4 + (size_t)2 * C * 2 + QT_STAGE_BYTES;
-  return qk_lds_bytes(ntab, C);
+  return layout == QK_LAYOUT_DMAJOR ? qt_lds_bytes(ntab, C, QT_TILE) : qk_lds_bytes(ntab, C);
 }
 size_t qk_norm_rope_lds_limit() { return LDS_LIMIT; }
 int qk_norm_rope_dmajor_max_dim() { return QT_MAX_NCH * 64 * 8; }
@@ -330,7 +332,7 @@ qk_norm_rope_kernel(const QkNormRopeArgs a) {
 }
 
 // ---------------------------------------------------------------- d-major layout
-// One workgroup of W waves per (tile of QT_ROWS tokens, tensor), each wave R = QT_ROWS / W token
+// One workgroup of W waves per (tile of TILE tokens, tensor), each wave R = TILE / W token
 // rows of it, their loads in flight while the vectors and tables fill the LDS. A 512-column slice
 // of the results is staged as rows, and each wave then writes CW columns of it: the LDS transpose read
 // (ds_read_b64_tr_b16: lane i of a 16-lane group gets four tokens of column i) gives a lane 8 or 16
@@ -341,31 +343,32 @@ qk_norm_rope_kernel(const QkNormRopeArgs a) {
 // 40 heads) and the memory in turn: the two workgroups of a CU mostly load, compute and store at
 // the same time. W = 8 lets two workgroups share a CU; a workgroup alone on its CU is bound by the
 // rate at which a wave issues, and takes W = 16 (launch_nch).
-template <int NCH, int W>
+template <int NCH, int W, int TILE>
 __global__ void __launch_bounds__(W * 64, 4)
 qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
-  constexpr int R = QT_ROWS / W;          // token rows per wave
+  constexpr int R = TILE / W;             // token rows per wave
+  constexpr int PPC = TILE / 8;           // 16-byte pieces of a column
   constexpr int CW = 512 / W;             // columns of a slice that one wave writes
-  constexpr int NP = CW * QT_PPC / 64;    // pieces per lane and slice
+  constexpr int NP = CW * PPC / 64;       // pieces per lane and slice
   constexpr int CG = CW / 16;             // 16-column groups of a wave
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int C = a.C;
   const int nchunk = C / 8;
   const int ntens = a.k != nullptr ? 2 : 1;
   // item numbering: XCD x (= blockIdx % 8) takes items [x * per, (x + 1) * per)
-  const int nitem = (a.L + QT_ROWS - 1) / QT_ROWS * ntens;
+  const int nitem = (a.L + TILE - 1) / TILE * ntens;
   const int per = (nitem + 7) / 8;
   const int item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (item >= nitem) return;  // whole workgroup, before any barrier
   const int t = item % ntens;
-  const int t0 = item / ntens * QT_ROWS;
-  const int nvalid = min(QT_ROWS, a.L - t0);
+  const int t0 = item / ntens * TILE;
+  const int nvalid = min(TILE, a.L - t0);
 
-  // LDS: [tables][bias, gamma of the tensor][2 stage buffers of QT_ROWS rows]
+  // LDS: [tables][bias, gamma of the tensor][2 stage buffers of TILE rows]
   float* tab = smem;
   uint16_t* vec = reinterpret_cast<uint16_t*>(smem + qk_table_floats(a.ntab));
   uint16_t* stage = vec + 2 * C;
-  constexpr int SB = QT_ROWS * QT_PITCH;  // one stage buffer
+  constexpr int SB = TILE * QT_PITCH;     // one stage buffer
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -409,8 +412,8 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
       qk_one_norm<NCH>(a, tab, u, t0 + wave + W * k, lane, s[k]);
 
   // the writing: per slice the wave's CW columns, as 16-byte pieces (8 tokens of a column)
-  // numbered column by column, QT_PPC to a column. A lane's transpose reads give it NP pieces of
-  // column rcol; piece id goes to chunk ((id / 4) % QT_ROWS, id % 4 + 4 (id / (4 QT_ROWS))) of the
+  // numbered column by column, PPC to a column. A lane's transpose reads give it NP pieces of
+  // column rcol; piece id goes to chunk ((id / 4) % TILE, id % 4 + 4 (id / (4 TILE))) of the
   // wave's part of the stage and is stored from there by lane id % 64.
   const int i16 = lane & 15, g = lane >> 4;
   const int rcol = 16 * (g % CG) + i16;
@@ -421,12 +424,12 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
   const int rd = lds_at(stage) + 2 * ((rtok + (i16 >> 2)) * QT_PITCH + CW * wave +
                                       16 * (g % CG) + 4 * (i16 & 3));
   auto piece_at = [&](int id) {  // element offset in a stage buffer
-    return (id / 4 % QT_ROWS) * QT_PITCH + CW * wave + 8 * (id % 4 + 4 * (id / (4 * QT_ROWS)));
+    return (id / 4 % TILE) * QT_PITCH + CW * wave + 8 * (id % 4 + 4 * (id / (4 * TILE)));
   };
   uint16_t* const out = t ? a.ko : a.qo;
   const int64_t os = t ? a.kos : a.qos;
-  const int ntok = nvalid - 8 * (lane % QT_PPC);  // tokens of this lane's pieces that exist (>= 8: all)
-  const int64_t lane_out = (int64_t)(lane / QT_PPC) * os + 8 * (lane % QT_PPC);
+  const int ntok = nvalid - 8 * (lane % PPC);  // tokens of this lane's pieces that exist (>= 8: all)
+  const int64_t lane_out = (int64_t)(lane / PPC) * os + 8 * (lane % PPC);
   const bool vec_ok = (t ? a.ko_vec : a.qo_vec) != 0;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -460,15 +463,15 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
     wave_lds_fence();
 #pragma unroll
     for (int j = 0; j < NP; ++j)
-      *reinterpret_cast<u32x4*>(sb + piece_at(rcol * QT_PPC + rtok / 8 + j)) =
+      *reinterpret_cast<u32x4*>(sb + piece_at(rcol * PPC + rtok / 8 + j)) =
           u32x4{x[2 * j][0], x[2 * j][1], x[2 * j + 1][0], x[2 * j + 1][1]};
     wave_lds_fence();
     if (vec_ok) {
 #pragma unroll
       for (int j = 0; j < NP; ++j) {
-        const int cj = col0 + 64 / QT_PPC * j;  // (wave-uniform) column of lane 0
+        const int cj = col0 + 64 / PPC * j;  // (wave-uniform) column of lane 0
         const u32x4 v = *reinterpret_cast<const u32x4*>(sb + piece_at(64 * j + lane));
-        if (cj + lane / QT_PPC >= C) continue;
+        if (cj + lane / PPC >= C) continue;
         uint16_t* dst = out + cj * os + t0 + lane_out;
         if (ntok >= 8) {
           *reinterpret_cast<u32x4*>(dst) = v;
@@ -480,9 +483,9 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
       }
     } else {
       // outputs that 16-byte stores cannot reach: consecutive lanes take consecutive tokens of a column
-      for (int e = lane; e < CW * QT_ROWS; e += 64) {
-        const int col = e / QT_ROWS, tok = e % QT_ROWS;
-        const uint16_t v = sb[piece_at(col * QT_PPC + tok / 8) + tok % 8];
+      for (int e = lane; e < CW * TILE; e += 64) {
+        const int col = e / TILE, tok = e % TILE;
+        const uint16_t v = sb[piece_at(col * PPC + tok / 8) + tok % 8];
         if (col0 + col < C && tok < nvalid) out[(int64_t)(col0 + col) * os + t0 + tok] = v;
       }
     }
@@ -497,16 +500,18 @@ qk_norm_rope_dmajor_kernel(const QkNormRopeArgs a) {
   }
 }
 
-template <int NCH, int W>
-static hipError_t launch_dmajor(const QkNormRopeArgs& a, int items, hipStream_t stream) {
+template <int NCH, int W, int TILE>
+static hipError_t launch_dmajor(const QkNormRopeArgs& a, hipStream_t stream) {
   static hipError_t attr = hipFuncSetAttribute(
-      (const void*)qk_norm_rope_dmajor_kernel<NCH, W>, hipFuncAttributeMaxDynamicSharedMemorySize,
-      (int)(qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR) < LDS_LIMIT
-                ? qk_norm_rope_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, QK_LAYOUT_DMAJOR)
+      (const void*)qk_norm_rope_dmajor_kernel<NCH, W, TILE>,
+      hipFuncAttributeMaxDynamicSharedMemorySize,
+      (int)(qt_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, TILE) < LDS_LIMIT
+                ? qt_lds_bytes(QK_MAX_TABLE, 64 * 8 * NCH, TILE)
                 : LDS_LIMIT));
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((qk_norm_rope_dmajor_kernel<NCH, W>), dim3(8 * ((items + 7) / 8)), dim3(W * 64),
-                     qk_norm_rope_lds_bytes(a.ntab, a.C, QK_LAYOUT_DMAJOR), stream, a);
+  const int items = (a.L + TILE - 1) / TILE * (a.k != nullptr ? 2 : 1);
+  hipLaunchKernelGGL((qk_norm_rope_dmajor_kernel<NCH, W, TILE>), dim3(8 * ((items + 7) / 8)),
+                     dim3(W * 64), qt_lds_bytes(a.ntab, a.C, TILE), stream, a);
   return hipGetLastError();
 }
 
@@ -525,13 +530,27 @@ static hipError_t launch_nch(const QkNormRopeArgs& a, int num_cus, hipStream_t s
       //   2560 x 40, 320 items, 34.6, 39.1; 3600, 450, 41.5, 45.8; 3600 x 24 26.8, 32.3.
       // - more items: 8 up to 8 chunks (10800 x 24 85, 92; x 32 108, 110), 16 for longer rows
       //   (4680 x 40 72.2, 64.6; 9360 119, 110; 10800 143, 128).
-      const int items = (a.L + QT_ROWS - 1) / QT_ROWS * (a.k != nullptr ? 2 : 1);
-      const bool pair = 2 * qk_norm_rope_lds_bytes(a.ntab, a.C, QK_LAYOUT_DMAJOR) <= LDS_LIMIT;
+      // - of these, rows of more than 6 chunks: 16 waves of two rows, tiles of 32 tokens, once a
+      //   round of them (39 us at 40 heads) costs less than the 16-token rounds (24 us) it replaces.
+      //   A line of the output gets 64 bytes from one workgroup instead of 32 each from two that
+      //   drift apart over the rounds. us for 32, 16 and (the form before all of these, one
+      //   workgroup of 16 waves per 16 tokens of both tensors): 7200 x 40 80, 99 (83); 8160 88, 105
+      //   (97); 10800 119, 128 (122); 14400 157, 178 (164); 7200 x 32 63, 74 (66); not 9360 x 40
+      //   119, 116 (116).
+      const int items = (a.L + QT_TILE - 1) / QT_TILE * (a.k != nullptr ? 2 : 1);
+      const bool pair = 2 * qt_lds_bytes(a.ntab, a.C, QT_TILE) <= LDS_LIMIT;
+      if constexpr (NCH > 6) {
+        const int items32 = (a.L + QT_LONG - 1) / QT_LONG * (a.k != nullptr ? 2 : 1);
+        const int rounds = (items + num_cus - 1) / num_cus;
+        const int rounds32 = (items32 + num_cus - 1) / num_cus;
+        if (items > 2 * num_cus && 3 * rounds > 5 * rounds32)
+          return launch_dmajor<NCH, 16, QT_LONG>(a, stream);
+      }
       if constexpr (NCH < 3 || NCH > 5) {
         if (items > num_cus && pair && (NCH < 9 || items <= 2 * num_cus))
-          return launch_dmajor<NCH, 8>(a, items, stream);
+          return launch_dmajor<NCH, 8, QT_TILE>(a, stream);
       }
-      return launch_dmajor<NCH, 16>(a, items, stream);
+      return launch_dmajor<NCH, 16, QT_TILE>(a, stream);
     }
   }
   static hipError_t attr = hipFuncSetAttribute((const void*)qk_norm_rope_kernel<NCH>,

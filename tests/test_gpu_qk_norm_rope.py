@@ -183,12 +183,14 @@ def test_dmajor_tiles_equal_rows(lib, L, C, cap):
 
 @pytest.mark.parametrize("C,L", [(256, 2061), (640, 2061), (1024, 4173), (3072, 2061), (3072, 4173),
                                  (3584, 2173), (4096, 2061), (4224, 2061), (4608, 4173),
-                                 (5120, 2061), (5120, 4173)])
+                                 (5120, 2061), (5120, 4173), (3584, 6205), (4224, 6205),
+                                 (5120, 6205)])
 @pytest.mark.parametrize("pad", [3, 6])
 def test_dmajor_many_tiles_equal_rows(lib, C, L, pad):
     """More (16-token tile, tensor) items than CUs, up to two per CU and beyond, with a partial last
-    tile: rows of every length class, two per wave and one, aligned and odd d strides, with the V
-    copy, both tensors and one (4173 tokens: above the CUs with one tensor as well)."""
+    tile: rows of every length class, two per wave and one, in tiles of 16 tokens and 32 (6205 with
+    both tensors), aligned and odd d strides, with the V copy, both tensors and one (from 4173 tokens
+    on above the CUs with one tensor as well)."""
     from lbw_amd import causal_rope_tables, qk_norm_rope_, wan_rope_freqs
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert 2 * ((L + 15) // 16) > cus and (L < 4000 or (L + 15) // 16 > cus)

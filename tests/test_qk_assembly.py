@@ -25,11 +25,11 @@ def asm():
 
 
 def _dmajor_kernels(asm):
-    """{(chunks, waves): lines} of the d-major kernel's instances."""
+    """{(chunks, waves, tile): lines} of the d-major kernel's instances."""
     out = {}
-    for m in re.finditer(r"^_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)E\S*:.*?^\.Lfunc_end",
+    for m in re.finditer(r"^_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)ELi(\d+)E\S*:.*?^\.Lfunc_end",
                          asm, re.M | re.S):
-        out[int(m.group(1)), int(m.group(2))] = m.group(0).splitlines()
+        out[tuple(int(g) for g in m.groups())] = m.group(0).splitlines()
     return out
 
 
@@ -56,22 +56,23 @@ def unfenced(lines):
 
 def test_lane_exchanges_are_fenced(asm):
     kernels = _dmajor_kernels(asm)
-    assert len(kernels) == 17  # 1..10 chunks per lane in 16 waves, all but 3..5 in 8
+    # 1..10 chunks per lane in 16 waves, all but 3..5 in 8; 7..10 with tiles of 32 tokens
+    assert len(kernels) == 21
     for inst, lines in kernels.items():
         assert any("ds_read_b64_tr" in l for l in lines), inst
         assert not unfenced(lines), inst
     # the check sees a missing fence: the same listing without either
-    lines = [l for l in kernels[6, 8] if "; wave barrier" not in l]
+    lines = [l for l in kernels[6, 8, 16] if "; wave barrier" not in l]
     assert unfenced(lines)
 
 
 def test_dmajor_kernels_use_no_scratch(asm):
     spilled = {}
     for block in re.split(r"^  - \.", asm, flags=re.M):
-        m = re.search(r"\.name: +_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)E", block)
+        m = re.search(r"\.name: +_ZN3lbw26qk_norm_rope_dmajor_kernelILi(\d+)ELi(\d+)ELi(\d+)E", block)
         if m:
-            spilled[int(m.group(1)), int(m.group(2))] = tuple(
+            spilled[m.groups()] = tuple(
                 int(re.search(rf"\.{key}: +(\d+)", block).group(1))
                 for key in ("private_segment_fixed_size", "vgpr_spill_count", "sgpr_spill_count"))
-    assert len(spilled) == 17
+    assert len(spilled) == 21
     assert all(v == (0, 0, 0) for v in spilled.values()), spilled
