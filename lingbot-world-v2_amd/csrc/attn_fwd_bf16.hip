@@ -978,11 +978,11 @@ attn_fwd_bf16_kernel(const AttnKernelArgs a) {
       } else {
         // P is packed in this block, not in the redo branch's successors
         asm volatile("" ::"v"(p_out[0]), "v"(p_out[1]), "v"(ls));
-        // softmax, part 3: a row sum beyond 2^16 (or not finite) means some p outgrew the
+        // softmax, part 3: a row sum beyond the limit (or not finite) means some p outgrew the
         // reference. Rare after a row's first tiles: move the reference to the row max of
         // this sub-block (and the old reference), redo the exponentials, and rescale O and l
         // by alpha like a tracked move. Exact either way: O and l share the reference.
-        if (__any(!(ls <= P_LIMIT))) {
+        if (__any(!(ls <= (TRACK ? P_LIMIT_TRACK : P_LIMIT)))) {
           float mx = s_in[0];
 #pragma unroll
           for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s_in[r]);

@@ -428,7 +428,7 @@ int run_chain(const lbw_attn_params* p, const float* so, const float* sm, const 
   const bool triple = p->part_o != nullptr;
   const size_t rows = (size_t)a.B * a.H * a.Lq;
   a.mode = kModePartials;
-  a.track_max = triple ? 1 : 0;  // the triple's m is the true row max; a normalised output needs none
+  a.track_max = 1;  // the triple's m is the true row max; the last call as accurate as the others
   if (!c.direct) {
     a.part_o = static_cast<float*>(ws);
     a.part_m = a.part_o + c.plan.splits * rows * p->head_dim;

@@ -167,6 +167,37 @@ def test_partials_match_oracle_and_merge(lib):
     assert_parity(merged, ref, "merge")
 
 
+@pytest.mark.parametrize("gain", [11.0, 14.0])
+def test_partials_follow_a_rise_below_overflow(lib, gain):
+    """One key whose score lies 2^10 to 2^15 above all earlier ones carries nearly the whole row.
+    The partials' reference moves to it, so its p is exactly 1 and O / l is off by the bf16 rounding
+    (2^-9 relative at most) of the other keys' p alone, plus 2^-17 for fp32. Against a reference left
+    at the earlier keys the large p itself would be rounded: up to 2^-9 of the row."""
+    from lbw_amd import attention_partial
+    g = torch.Generator().manual_seed(int(gain))
+    B, Lq, H, L, top = 1, 200, 3, 150, 100
+    u = torch.randn(128, generator=g)
+    u = u / u.norm()
+    rise = gain + 2.0 * torch.rand(B, Lq, H, 1, generator=g) - 1.0      # log2 units, a row each
+    q = (rise * u).to(torch.bfloat16)
+    k = torch.randn(B, L, H, 128, generator=g) * 0.01
+    k[:, top] = math.log(2.0) * math.sqrt(128) * u
+    k = k.to(torch.bfloat16)
+    v = torch.randn(B, L, H, 128, generator=g).to(torch.bfloat16)
+    po, _, pl = attention_partial(q.to(DEV), [(k.to(DEV), v.to(DEV))])
+    s = torch.einsum("blhd,bkhd->bhlk", q.double(), k.double()) / math.sqrt(128)
+    p = torch.softmax(s, dim=-1)
+    vd = v.double().permute(0, 2, 1, 3)
+    ref = p @ vd
+    rest = p.clone()
+    rest[..., top] = 0
+    assert float(p[..., top].min()) > 0.8
+    bound = 2.0 ** -9 * (rest @ vd.abs()) + 2.0 ** -17 * vd.abs().amax()
+    err = ((po / pl[..., None]).cpu().double() - ref).abs()
+    print(f"gain {gain}: worst error / bound {float((err / bound).max()):.3f}")
+    assert bool((err <= bound).all())
+
+
 def test_chain_over_key_sets_equals_union(lib):
     """cte_call's chain (attention.py:654-694): calls over the cached chunks, then the new
     chunk, continue one softmax; the normalizing call equals attention over all the keys."""
