@@ -18,6 +18,7 @@
 #include <torch/library.h>
 
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "lbw_attn.h"
@@ -336,6 +337,19 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attention_chain(
   return {part.o, part.m, part.l};
 }
 
+// Addresses [first, one past the last) of a tensor's elements (strides are not negative).
+std::pair<uintptr_t, uintptr_t> extent(const at::Tensor& t) {
+  const auto p = reinterpret_cast<uintptr_t>(t.data_ptr());
+  if (t.numel() == 0) return {p, p};
+  int64_t last = 0;
+  for (int64_t d = 0; d < t.dim(); ++d) last += (t.size(d) - 1) * t.stride(d);
+  return {p, p + (last + 1) * t.element_size()};
+}
+bool may_overlap(const at::Tensor& a, const at::Tensor& b) {
+  const auto x = extent(a), y = extent(b);
+  return x.first < y.second && y.first < x.second;
+}
+
 void attention_chain_out(const at::Tensor& q, at::TensorList k, at::TensorList v,
                          const std::optional<at::Tensor>& so, const std::optional<at::Tensor>& sm,
                          const std::optional<at::Tensor>& sl, int64_t kv_lo, int64_t kv_hi,
@@ -347,10 +361,23 @@ void attention_chain_out(const at::Tensor& q, at::TensorList k, at::TensorList v
                   out.stride(3) == 1 && out.device() == q.device(),
               "out must be bf16 [B, Lq, N, D] with a contiguous head dim");
   lbw_attn_params p = base_params(q, k, v, kv_lo, kv_hi, softmax_scale, 0);
+  // the call may write rows of out before it has read all of its inputs: an out that shares memory
+  // with one of them is filled by a copy at the end
+  bool shared = may_overlap(out, q);
+  for (size_t i = 0; i < k.size(); ++i) shared |= may_overlap(out, k[i]) || may_overlap(out, v[i]);
+  for (const auto* s : {&so, &sm, &sl}) shared |= s->has_value() && may_overlap(out, **s);
   set_out(p, out, q);
+  at::Tensor dst = out;
+  if (shared) {
+    TORCH_CHECK(q.size(1) == 0 || lbw_attention_chain_workspace_size(&p, so.has_value()) > 0,
+                "lbw_attention_chain: ", lbw_last_error());  // (out's own layout, as without it)
+    dst = at::empty(q.sizes(), out.options());
+    set_out(p, dst, q);
+  }
   DevBounds db;
   db.set(p, kv_lo_dev, kv_hi_dev, q);
   run_chain(p, q, so, sm, sl, nullptr);
+  if (shared) out.copy_(dst);
 }
 
 void attention_merge_out(at::TensorList o, at::TensorList m, at::TensorList l,

@@ -512,6 +512,36 @@ def test_chain_calls_cut_into_pieces(lib, H, Lq, lens, scale):
     assert torch.all(wide[..., 128:] == 0)
 
 
+@pytest.mark.parametrize("shares", ["k", "v", "q", "state"])
+@pytest.mark.parametrize("H,Lq,keys", [(3, 300, 1100), (40, 700, 800)])
+def test_chain_out_may_share_memory_with_an_input(lib, H, Lq, keys, shares):
+    """The normalising call with an ``out`` that lies in K's, V's, q's (strided otherwise) or the
+    state's memory gives what it gives into memory of its own: as a chain's only call (rows of out
+    are written while other rows' keys are still read) and after another."""
+    from lbw_amd import attention_chain
+    q, ks, vs = _case(1, Lq, H, [keys, 200], seed=H, gain=False)
+
+    def run(shared):
+        buf = {"k": ks[0].to(DEV), "v": vs[0].to(DEV),
+               "q": torch.zeros(1, Lq, H, 256, dtype=torch.bfloat16, device=DEV)}
+        qd = buf["q"][..., :128]
+        qd.copy_(q)
+        state = None
+        if shares == "state":
+            state = attention_chain(qd, [(ks[1].to(DEV), vs[1].to(DEV))])
+            buf["state"] = state[0]
+        out = torch.empty(1, Lq, H, 128, dtype=torch.bfloat16, device=DEV)
+        if shared:   # the same number of rows of 128, from the start of that tensor's memory
+            flat = buf[shares].view(-1) if shares != "state" else buf["state"].view(-1).view(torch.bfloat16)
+            out = flat[:out.numel()].view(out.shape)
+        got = attention_chain(qd, [(buf["k"], buf["v"])], state, normalize=True, out=out)
+        torch.cuda.synchronize()
+        assert got.data_ptr() == out.data_ptr()
+        return got.clone()
+
+    assert torch.equal(run(True), run(False))
+
+
 def test_chain_refuses_a_wrong_state(lib):
     from lbw_amd import attention_chain
     q, ks, vs = _case(1, 40, 2, [100], seed=1)
