@@ -187,12 +187,13 @@ int lbw_attn_merge_partials(int32_t n_parts, const float* const* part_o,
 /* One call of cte_call's chain (wan/modules/attention.py:654-694): attention over the params' KV
  * segments joined with the running triple of the earlier calls (state_o [B, H, Lq, D], state_m and
  * state_l [B, H, Lq], fp32, contiguous; all three NULL for a chain's first call). With part_o,
- * part_m and part_l the new triple is written there (m the true row max; it must not overlap the
- * state); without them the chain ends and `out` gets the normalised result. The results are those
- * of lbw_attention_fwd's partials and lbw_attn_merge_partials / lbw_attn_merge up to fp32
- * rounding; the call's keys may be cut into pieces that run side by side (num_splits: 0 = the
- * host's choice, up to 15). The workspace holds the pieces' partials and, as for
- * lbw_attention_fwd, backs one in-flight call. */
+ * part_m and part_l the new triple is written there (m the true row max; one that overlaps the
+ * state is refused); without them the chain ends and `out` gets the normalised result. `out` must
+ * not overlap q, the keys and values or the state: rows of it may be written before all of these
+ * are read. The results are those of lbw_attention_fwd's partials and lbw_attn_merge_partials /
+ * lbw_attn_merge up to fp32 rounding; the call's keys may be cut into pieces that run side by side
+ * (num_splits: 0 = the host's choice, up to 15; more ask for 15). Not with a key_bias. The
+ * workspace holds the pieces' partials and, as for lbw_attention_fwd, backs one in-flight call. */
 size_t lbw_attention_chain_workspace_size(const lbw_attn_params* p, int32_t has_state);
 int lbw_attention_chain(const lbw_attn_params* p, const float* state_o, const float* state_m,
                         const float* state_l, void* workspace, size_t workspace_bytes,

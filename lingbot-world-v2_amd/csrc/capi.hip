@@ -416,6 +416,19 @@ int run_chain(const lbw_attn_params* p, const float* so, const float* sm, const 
   ChainPlan c;
   int rc = make_chain_plan(p, state, &c);
   if (rc != LBW_OK) return rc;
+  if (state && p->part_o != nullptr) {
+    // one thread of the merge writes a row's m and l while others still read the state's
+    const size_t n = (size_t)p->batch * p->heads * p->lq * sizeof(float);
+    const std::pair<const float*, size_t> in[3] = {{so, n * p->head_dim}, {sm, n}, {sl, n}};
+    const std::pair<const float*, size_t> out[3] = {{p->part_o, n * p->head_dim}, {p->part_m, n},
+                                                    {p->part_l, n}};
+    for (const auto& x : in)
+      for (const auto& y : out) {
+        const auto a = reinterpret_cast<uintptr_t>(x.first), b = reinterpret_cast<uintptr_t>(y.first);
+        if (a < b + y.second && b < a + x.second)
+          return fail(LBW_ERR_INVALID, "the new triple overlaps the state");
+      }
+  }
   if (c.plain) return run_attention(p, false, ws, ws_bytes, stream);
   if (p->lq == 0) return LBW_OK;
   AttnKernelArgs& a = c.plan.a;

@@ -228,6 +228,47 @@ def test_workspace_layout_without_gpu():
             (H, LQ, LK, n, splits)
 
 
+def test_chain_refuses_a_triple_over_the_state_without_gpu():
+    """The merge reads a row of the state while it writes the new triple: any overlap of the two is
+    refused before any HIP call, neighbours are not."""
+    from lbw_amd import _lib
+    lib = _lib.load()
+    B, H, LQ = 1, 2, 64
+    p = _lib.AttnParams()
+    p.batch, p.heads, p.head_dim, p.lq = B, H, 128, LQ
+    p.q = 1 << 30
+    p.q_stride_b, p.q_stride_l, p.q_stride_h = LQ * H * 128, H * 128, 128
+    p.n_segments = 1
+    s = p.seg[0]
+    s.k = s.v = 1 << 31
+    s.len = 64
+    s.k_stride_b = s.v_stride_b = 64 * H * 128
+    s.k_stride_l = s.v_stride_l = H * 128
+    s.k_stride_h = s.v_stride_h = 128
+    p.kv_lo, p.kv_hi = 0, -1
+    row, big = B * H * LQ * 4, B * H * LQ * 128 * 4
+    so, sm, sl = 1 << 20, 1 << 24, 1 << 25
+    apart = (1 << 26, 1 << 27, 1 << 28)
+
+    def call(po, pm, pl):
+        p.part_o, p.part_m, p.part_l = po, pm, pl
+        rc = lib.lbw_attention_chain(ctypes.byref(p), so, sm, sl, None, 0, None)
+        return rc, lib.lbw_last_error()
+
+    for i, x in ((0, so), (0, so + big - 16), (0, so - big + 16), (1, sm), (1, sl + 4),
+                 (2, sl + row - 4), (1, so + big - 4), (0, sm + row - 16)):
+        parts = list(apart)
+        parts[i] = x
+        rc, msg = call(*parts)
+        assert rc == 1 and b"overlaps" in msg, (i, x - so)
+    # next to the state but not over it: past this check, to the missing workspace
+    for i, x in ((0, so + big), (0, so - big), (1, sm + row), (2, sl - row)):
+        parts = list(apart)
+        parts[i] = x
+        rc, msg = call(*parts)
+        assert rc == 4 and b"workspace" in msg, (i, msg)
+
+
 def test_segment_length_limit_without_gpu():
     """Segments longer than 2^30 keys are refused before any HIP call (32-bit key indices)."""
     from lbw_amd import _lib
@@ -284,7 +325,8 @@ def test_torch_op_set_registers_with_shapes():
     ops = _lib.ops()
     for name in ("attention", "attention_out", "cross_attention", "cross_attention_out",
                  "attention_fp8kv", "attention_fp8kv_out", "attention_partial",
-                 "attention_merge", "attention_merge_out", "qk_norm_rope_", "kv_quant_fp8_"):
+                 "attention_merge", "attention_merge_out", "attention_chain",
+                 "attention_chain_out", "qk_norm_rope_", "kv_quant_fp8_"):
         assert hasattr(ops, name), name
     q = torch.empty(2, 10, 3, 128, dtype=torch.bfloat16, device="meta")
     k = torch.empty(2, 70, 3, 128, dtype=torch.bfloat16, device="meta")
@@ -295,6 +337,9 @@ def test_torch_op_set_registers_with_shapes():
     po, pm, pl = ops.attention_partial(q, [k], [k], 0, -1, 0.0)
     assert po.shape == (2, 3, 10, 128) and pm.shape == (2, 3, 10) and pl.dtype == torch.float32
     assert ops.attention_merge([po, po], [pm, pm], [pl, pl]).shape == q.shape
+    co, cm, cl = ops.attention_chain(q, [k], [k], po, pm, pl, 0, -1, 0.0)
+    assert co.shape == po.shape and cm.shape == cl.shape == pm.shape and co.dtype == torch.float32
+    ops.attention_chain_out(q, [k], [k], None, None, None, 0, -1, 0.0, torch.empty_like(q))
     c8 = torch.empty(2, 70, 3, 128, dtype=torch.uint8, device="meta")
     s8 = torch.empty(2, 3, 2, dtype=torch.float32, device="meta")
     assert ops.attention_fp8kv(q, [c8], [c8], [s8], [s8], 0, -1, 0.0, 0, False).shape == q.shape
