@@ -44,3 +44,12 @@ def cosine(a, b) -> float:
     a = a.detach().double().flatten().cpu()
     b = b.detach().double().flatten().cpu()
     return float((a @ b) / (a.norm() * b.norm()))
+
+
+def more_items_than_cus(B, H, Lq, splits) -> bool:
+    """Whether a chunk-kernel call has more work items (batch x head x 256-query tile, times the
+    pieces) than the GPU has CUs: then they go through the work queues, and 2 to 8 pieces merge in
+    the kernel; else each item has a CU of its own and pieces merge in a launch of their own."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return B * H * ((Lq + 255) // 256) * max(splits, 1) > cus

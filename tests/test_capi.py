@@ -199,12 +199,15 @@ def _split_count(H, LQ, LK):
 
 def test_workspace_layout_without_gpu():
     """Workspace = split partials (splits x rows x (D + 2) fp32) rounded up to 256 bytes, then
-    the counters: 8 work-queue counters and, for a split plan (its pieces merge in the kernel),
-    one arrival counter per (batch, head, 256-query tile), rounded up to 256 bytes (at least
-    256); a single-pass plan needs only the queue counters."""
+    the counters: 8 work-queue counters and, for a plan whose pieces merge in the kernel (2 to 8
+    of them, with more work items than CUs), one arrival counter per (batch, head, 256-query tile),
+    rounded up to 256 bytes (at least 256); the others need only the queue counters."""
+    import torch
     from lbw_amd import _lib
     lib = _lib.load()
-    for H, LQ, LK in [(2, 256, 1024), (40, 3600, 46800), (40, 4680, 32760), (12, 4680, 14040)]:
+    cus = torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available() else 256
+    for H, LQ, LK in [(2, 256, 1024), (40, 3600, 46800), (40, 4680, 32760), (12, 4680, 14040),
+                      (12, 1560, 4680)]:     # the last: 84 units in 3 pieces, a CU for each
         p = _lib.AttnParams()
         p.batch, p.heads, p.head_dim, p.lq = 1, H, 128, LQ
         p.q = p.out = 256
@@ -223,7 +226,7 @@ def test_workspace_layout_without_gpu():
         splits = _split_count(H, LQ, LK)
         parts = splits * LQ * H * 130 * 4 if splits > 1 else 0
         units = H * ((LQ + 255) // 256)
-        cnt = 4 * (8 + (units if splits > 1 else 0))
+        cnt = 4 * (8 + (units if 1 < splits <= 8 and units * splits > cus else 0))
         assert n == ((parts + 255) // 256) * 256 + max(256, (cnt + 255) // 256 * 256), \
             (H, LQ, LK, n, splits)
 

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle as O
-from parity import assert_parity, metrics
+from parity import assert_parity, metrics, more_items_than_cus
 
 pytestmark = pytest.mark.gpu
 
@@ -102,18 +102,27 @@ def test_split_kv_merge_matches_single_pass(lib, splits):
     assert (one.float() - many.float()).abs().max() < 4e-3
 
 
-@pytest.mark.parametrize("B,Lq,H,Lk,splits", [
-    (1, 40, 1, 700, 3),      # one unit: seven XCD queues empty, their workgroups take from XCD 0
-    (1, 300, 3, 900, 2),     # six units, ragged last q-tile
-    (2, 513, 3, 333, 5),     # batch 2, 18 units, pieces of 1-2 tiles
-    (1, 256, 5, 130, 7),     # more pieces than tiles: empty pieces merge as nothing
-    (3, 100, 7, 2000, 1),    # 21 units, single pass through the queues
+@pytest.mark.parametrize("B,Lq,H,Lk,splits,queued", [
+    # a CU per item: fixed items (an eighth per XCD), pieces merged in their own launch
+    (1, 40, 1, 700, 3, False),      # one unit
+    (1, 300, 3, 900, 2, False),     # six units, ragged last q-tile
+    (2, 513, 3, 333, 5, False),     # batch 2, 18 units, pieces of 1-2 tiles
+    (1, 256, 5, 130, 7, False),     # more pieces than tiles: empty pieces merge as nothing
+    (3, 100, 7, 2000, 1, False),    # 21 units, single pass
+    # more items than CUs: the queues, and up to 8 pieces merged in the kernel
+    (1, 40, 130, 700, 3, True),     # ragged short rows
+    (2, 40, 65, 500, 5, True),      # batch 2, pieces of 1-2 tiles
+    (1, 300, 43, 900, 4, True),     # 86 units: not a multiple of the XCDs
+    (1, 256, 45, 130, 7, True),     # more pieces than tiles: empty pieces arrive as well
+    (3, 100, 87, 300, 1, True),     # single pass
+    (1, 33, 37, 800, 12, True),     # pieces merged in their own launch
 ])
-def test_work_queue_covers_every_item(lib, B, Lq, H, Lk, splits):
-    """The per-XCD work queues with stealing hand every (piece, batch, head, q-tile) item to
-    exactly one workgroup for unit counts below, at and above the XCD count, with pieces that
-    hold no tiles, and with batch > 1."""
+def test_work_queue_covers_every_item(lib, B, Lq, H, Lk, splits, queued):
+    """Every (piece, batch, head, q-tile) item is run by exactly one workgroup, whether each has a
+    CU of its own or the per-XCD work queues with stealing hand them out: unit counts below, at and
+    above the XCD count and not multiples of it, pieces that hold no tiles, batch > 1."""
     from lbw_amd import attention_segments
+    assert more_items_than_cus(B, H, Lq, splits) == queued
     q, ks, vs = _case(B, Lq, H, [Lk], seed=B * 1000 + Lq + splits)
     # V halved (exact in bf16): with a few hundred keys a peaked head copies single V rows, and
     # |o| >= 4 would put one bf16 output rounding above the 1e-2 bound
@@ -317,13 +326,15 @@ def test_torch_ops_refuse_wrong_types_and_shapes(lib):
     torch.cuda.synchronize()
 
 
-def test_two_streams_get_separate_workspaces(lib):
-    """Two split-KV calls in flight on two streams at once: each call's workspace (work-queue
-    counters and partials) comes from the caching allocator on its own stream, so neither call
-    takes the other's items or overwrites its partials. Both outputs are checked against the
-    oracle."""
+@pytest.mark.parametrize("H,queued", [(3, False), (30, True)])
+def test_two_streams_get_separate_workspaces(lib, H, queued):
+    """Two split-KV calls in flight on two streams at once: each call's workspace (partials and,
+    with more items than CUs, the counters of its work queues and arrivals) comes from the caching
+    allocator on its own stream, so neither call takes the other's items or overwrites its partials.
+    Both outputs are checked against the oracle."""
     from lbw_amd import attention_segments
-    cases = [_case(1, 700, 3, [3000], seed=s) for s in (31, 32)]
+    assert more_items_than_cus(1, H, 700, 4) == queued
+    cases = [_case(1, 700, H, [3000], seed=s, gain=H == 3) for s in (31, 32)]
     dev_in = [(q.to(DEV), ks[0].to(DEV), vs[0].to(DEV)) for q, ks, vs in cases]
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
     cur = torch.cuda.current_stream()

@@ -1,22 +1,24 @@
 """The hot path under the two ways a PyTorch program hands it to the runtime as a whole:
 
 - HIP graphs: the per-layer chunk step (fused q/k RMSNorm + RoPE writing the pre-scaled q and the
-  chunk's K/V into its cache slot, then the folded-softmax attention with split pieces, work
-  queues and the merge) captured once and replayed with new inputs, with eager work and
-  synchronisations between the replays; every replay is checked bitwise against an eager run of
-  the same step (the kernels are deterministic: the work queues change which workgroup runs an
-  item, not what it computes). The work-queue counters are cleared by a kernel, not a memset, so
-  the captured graph stays correct on every replay.
+  chunk's K/V into its cache slot, then the folded-softmax attention with split pieces) captured
+  once and replayed with new inputs, with eager work and synchronisations between the replays;
+  every replay is checked bitwise against an eager run of the same step (the kernels are
+  deterministic: the work queues change which workgroup runs an item, not what it computes). With
+  4 heads each item has a CU of its own and the merge its own launch; with 40 the items go through
+  the work queues and merge in the kernel, whose counters a kernel clears, not a memset, so the
+  captured graph stays correct on every replay.
 - torch.compile: the `torch.ops.lbw` operators carry Meta implementations, so a function calling
   them traces as one graph (fullgraph=True fails on any graph break) and gives the eager results.
 """
 import pytest
 import torch
 
+from parity import more_items_than_cus
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-H, D = 4, 128
-C = H * D
+D = 128
 GRID = (1, 20, 30)            # 600 tokens per chunk
 LQ = GRID[0] * GRID[1] * GRID[2]
 CACHED = 3                    # frames before the chunk
@@ -25,6 +27,8 @@ LK = LQ * (CACHED + 1)
 
 def _step(bufs, tabs):
     from lbw_amd import PRESCALED_SOFTMAX_SCALE, attention_segments, prescaled_q_scale, qk_norm_rope_
+    C = bufs["q"].shape[1]
+    H = C // D
     slot = slice(LK - LQ, LK)
     qk_norm_rope_(bufs["xq"], bufs["xk"], None, None, bufs["wq"], bufs["wk"], tabs, 1e-6, H,
                   q_out=bufs["q"], k_out=bufs["ck"][0, slot].view(LQ, C), v=bufs["xv"],
@@ -33,7 +37,8 @@ def _step(bufs, tabs):
                        softmax_scale=PRESCALED_SOFTMAX_SCALE, num_splits=3)
 
 
-def _buffers(g):
+def _buffers(g, H):
+    C = H * D
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
     return dict(xq=rnd(LQ, C), xk=rnd(LQ, C), xv=rnd(LQ, C),
                 wq=(1 + 0.1 * torch.randn(C, generator=g, device=DEV)).to(torch.bfloat16),
@@ -43,11 +48,13 @@ def _buffers(g):
                 out=torch.empty(1, LQ, H, D, dtype=torch.bfloat16, device=DEV))
 
 
-def test_hip_graph_replays_the_chunk_step(lib):
+@pytest.mark.parametrize("H,queued", [(4, False), (40, True)])
+def test_hip_graph_replays_the_chunk_step(lib, H, queued):
     from lbw_amd import causal_rope_tables, wan_rope_freqs
+    assert more_items_than_cus(1, H, LQ, 3) == queued
     g = torch.Generator(device=DEV).manual_seed(3)
     tabs = causal_rope_tables(wan_rope_freqs(D), GRID, CACHED, device=DEV)
-    static = _buffers(g)
+    static = _buffers(g, H)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):   # warm-up off the capture stream, as torch requires
@@ -59,7 +66,7 @@ def test_hip_graph_replays_the_chunk_step(lib):
     torch.cuda.synchronize()
     for rep in range(3):
         print(f"replay {rep}", flush=True)
-        fresh = _buffers(g)
+        fresh = _buffers(g, H)
         for name in ("xq", "xk", "xv", "wq", "wk", "ck", "cv"):
             static[name].copy_(fresh[name])
         graph.replay()
@@ -77,6 +84,7 @@ def test_hip_graph_replays_the_chunk_step(lib):
 def test_torch_compile_traces_the_ops_as_one_graph(lib):
     from lbw_amd import _lib
     _lib.ops()  # registers torch.ops.lbw
+    H = 4
     g = torch.Generator(device=DEV).manual_seed(4)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
     q, k, v = rnd(1, 300, H, D), rnd(1, 1000, H, D), rnd(1, 1000, H, D)
@@ -100,7 +108,7 @@ def test_torch_compile_traces_the_ops_as_one_graph(lib):
 
 def _xstep(b):
     """Cross-attention to a masked context, then the fp8-KV path: the quantiser and the fp8
-    attention over 3 pieces (work queues and merge); returns both outputs."""
+    attention over 3 pieces; returns both outputs."""
     from lbw_amd import attention_fp8kv, cross_attention, quantize_kv_fp8
     x = cross_attention(b["q"], b["kc"], b["vc"], k_lens=b["kl"])
     k8, v8 = quantize_kv_fp8(b["k"]), quantize_kv_fp8(b["v"])
@@ -108,20 +116,22 @@ def _xstep(b):
     return x, y
 
 
-def _xbuffers(g, valid):
+def _xbuffers(g, valid, H):
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
     return dict(q=rnd(1, LQ, H, D), kc=rnd(1, 512, H, D), vc=rnd(1, 512, H, D),
                 kl=torch.tensor([valid], dtype=torch.int32, device=DEV),
                 k=rnd(1, 1500, H, D), v=rnd(1, 1500, H, D))
 
 
-def test_hip_graph_replays_cross_and_fp8(lib):
+@pytest.mark.parametrize("H,queued", [(4, False), (40, True)])
+def test_hip_graph_replays_cross_and_fp8(lib, H, queued):
     """The cross-attention kernel and the fp8-KV path (quantiser, fp8 attention with split
-    pieces, work queues, merge) captured once and replayed with new inputs -- a new valid
-    context length read by the kernel from the device each replay included -- each replay
-    bitwise equal to an eager run between the replays."""
+    pieces and their merge, with 40 heads through the work queues) captured once and replayed with
+    new inputs -- a new valid context length read by the kernel from the device each replay
+    included -- each replay bitwise equal to an eager run between the replays."""
+    assert more_items_than_cus(1, H, LQ, 3) == queued
     g = torch.Generator(device=DEV).manual_seed(5)
-    static = _xbuffers(g, 300)
+    static = _xbuffers(g, 300, H)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -133,7 +143,7 @@ def test_hip_graph_replays_cross_and_fp8(lib):
     torch.cuda.synchronize()
     for rep, valid in enumerate((300, 77, 512)):
         print(f"replay {rep}: {valid} valid context rows", flush=True)
-        fresh = _xbuffers(g, valid)
+        fresh = _xbuffers(g, valid, H)
         for name in ("q", "kc", "vc", "kl", "k", "v"):
             static[name].copy_(fresh[name])
         graph.replay()

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import oracle as O
-from parity import assert_parity, metrics
+from parity import assert_parity, metrics, more_items_than_cus
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -54,6 +54,29 @@ def test_dmajor_k_matches_oracle(lib, B, Lq, H, lens, window, splits):
     assert_parity(out, ref)
     # the same products summed in another order inside the MFMA: one bf16 step at most
     assert float((out.float() - tok.float()).abs().max()) <= 2.0 ** -6 * max(1.0, float(tok.float().abs().max()))
+
+
+@pytest.mark.parametrize("B,Lq,H,lens,window,splits", [
+    (1, 300, 33, [1000, 600], None, 4),             # 264 items, merged in the kernel
+    (2, 129, 40, [104, 40, 200, 8], (50, 300), 5),  # pieces of one tile and none
+    (1, 40, 264, [136], None, 1),                   # single pass
+])
+def test_dmajor_k_more_items_than_cus(lib, B, Lq, H, lens, window, splits):
+    """The same through the work queues and the in-kernel merge."""
+    assert more_items_than_cus(B, H, Lq, splits)
+    test_dmajor_k_matches_oracle(lib, B, Lq, H, lens, window, splits)
+
+
+def test_dmajor_k_prescaled_more_items_than_cus(lib):
+    """The folded softmax over d-major K through the work queues and the in-kernel merge."""
+    from lbw_amd import PRESCALED_SOFTMAX_SCALE, attention_segments, prescaled_q_scale
+    q, ks, vs = _case(1, 200, 90, [600, 344], seed=9)
+    assert more_items_than_cus(1, 90, 200, 3)
+    qs = (q.float() * prescaled_q_scale(128)).to(torch.bfloat16)
+    segs = [(_dmajor(k), v.to(DEV)) for k, v in zip(ks, vs)]
+    out = attention_segments(qs.to(DEV), segs, softmax_scale=PRESCALED_SOFTMAX_SCALE, num_splits=3)
+    assert_parity(out, O.attention_ref(qs, torch.cat(ks, 1), torch.cat(vs, 1),
+                                       softmax_scale=math.log(2.0)), "folded")
 
 
 def test_dmajor_k_prescaled_and_partials(lib):

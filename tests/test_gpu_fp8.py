@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import oracle as O
-from parity import FP8_COSINE, cosine, metrics
+from parity import FP8_COSINE, cosine, metrics, more_items_than_cus
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -251,8 +251,25 @@ def test_fp8_kernel_arithmetic_fp32(lib, Lq, H, lk, window, splits):
     assert rel_l1 <= 4e-3
 
 
+@pytest.mark.parametrize("Lq,H,lk,window,splits", [
+    (40, 66, 700, None, 4),          # 264 items, merged in the kernel
+    (290, 40, 330, (3, 329), 8),     # more pieces than tiles, two q-tiles
+    (33, 264, 130, None, 1),         # single pass
+])
+def test_fp8_more_items_than_cus(lib, Lq, H, lk, window, splits):
+    """The same through the work queues and the in-kernel merge."""
+    assert more_items_than_cus(1, H, Lq, splits)
+    test_fp8_kernel_arithmetic_fp32(lib, Lq, H, lk, window, splits)
+
+
+@pytest.mark.parametrize("n_segs,splits,H", [(1, 4, 40), (2, 3, 50)])
+def test_fp8_prescaled_more_items_than_cus(lib, n_segs, splits, H):
+    assert more_items_than_cus(1, H, 290, splits)
+    test_fp8_prescaled_q_folded(lib, n_segs, splits, H)
+
+
 @pytest.mark.parametrize("n_segs,splits", [(1, 0), (1, 3), (2, 0), (2, 2)])
-def test_fp8_prescaled_q_folded(lib, n_segs, splits):
+def test_fp8_prescaled_q_folded(lib, n_segs, splits, H=3):
     """A q pre-scaled by log2(e)/sqrt(d) with softmax scale ln 2 takes the folded fp8 instances
     (one segment: tile copies addressed by index; two: the general cursor): the fp32 output
     against the oracle on the dequantised K/V within the kernel's arithmetic bound, and within
@@ -261,7 +278,7 @@ def test_fp8_prescaled_q_folded(lib, n_segs, splits):
     from lbw_amd import (PRESCALED_SOFTMAX_SCALE, attention_fp8kv, prescaled_q_scale,
                          quantize_kv_fp8)
     g = torch.Generator().manual_seed(31 + n_segs + splits)
-    H, Lq = 3, 290
+    Lq = 290
     lens = (1300,) if n_segs == 1 else (640, 130)
     q = _wide_q(Lq, H, g)
     qs = (q.float() * prescaled_q_scale(128)).to(torch.bfloat16)

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle as O
-from parity import assert_parity
+from parity import assert_parity, more_items_than_cus
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -34,9 +34,12 @@ def _noalloc(lib, q, k, v, splits):
 
 def test_noalloc_matches_allocating_entry_point(lib):
     from lbw_amd import attention_segments
-    # (B, Lq, H, keys, splits): a split call whose partials fill 33 MB of the scratch, then a
+    # (B, Lq, H, keys, splits): a split call whose partials fill 33 MB of the scratch (a CU per
+    # item) and one of 37 MB with more items than CUs (work queues, in-kernel merge), each before a
     # smaller one with the host's own split choice
-    for B, Lq, H, L, splits in [(1, 2000, 8, 6000, 4), (2, 700, 3, 3000, 0)]:
+    assert more_items_than_cus(1, 9, 2000, 4)
+    for B, Lq, H, L, splits in [(1, 2000, 8, 6000, 4), (2, 700, 3, 3000, 0),
+                                (1, 2000, 9, 6000, 4), (2, 700, 3, 3000, 0)]:
         q, k, v = _inputs(B, Lq, H, L, seed=Lq)
         qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
         print(f"case B={B} Lq={Lq} H={H} keys={L} splits={splits}", flush=True)
@@ -79,14 +82,17 @@ def test_noalloc_lowers_the_host_split_choice_to_what_fits(lib):
     assert not torch.equal(out, other)
 
 
-def test_noalloc_replays_in_a_hip_graph(lib):
-    """The entry point captured in a HIP graph (its queue counters are cleared by a kernel, not
-    a memset) and replayed with new inputs, every replay bitwise equal to an eager call of the
-    allocating entry point, with eager work between the replays."""
+@pytest.mark.parametrize("H,queued", [(6, False), (40, True)])
+def test_noalloc_replays_in_a_hip_graph(lib, H, queued):
+    """The entry point captured in a HIP graph and replayed with new inputs, every replay bitwise
+    equal to an eager call of the allocating entry point, with eager work between the replays: with
+    a CU per item, and through the work queues, whose counters are cleared by a kernel, not a
+    memset."""
     from lbw_amd import _lib, attention_segments
+    assert more_items_than_cus(1, H, 700, 3) == queued
     g = torch.Generator(device=DEV).manual_seed(3)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
-    q, k, v = rnd(1, 700, 6, 128), rnd(1, 4000, 6, 128), rnd(1, 4000, 6, 128)
+    q, k, v = rnd(1, 700, H, 128), rnd(1, 4000, H, 128), rnd(1, 4000, H, 128)
     out = torch.empty_like(q)
     p = _lib.attn_params(q, out, [(k, v)], None, None, None, None, 3)
     side = torch.cuda.Stream()
