@@ -64,6 +64,7 @@ int num_cus() {
 // near equals. Fitted to measured gfx950 times, in
 // us, of 1, 2, 3, .. pieces: 40 heads x 3600 q x 3600 keys 267, 290, 325; 10 x 3600 x 46800 850,
 // 969, 745, 790, 725, 773; 12 x 1560 x 4680 100, 70, 60, 82; 12 x 4680 x 14040 343, 364, 373.
+// (By itself a one-wave item of a long call measured 0.72 of a full one, not the 0.39 used here.)
 double split_cost(int64_t bh, int lq, int bm, int64_t ntiles, int s, int cus) {
   const int nq = (lq + bm - 1) / bm;
   const int tail_q = lq - (nq - 1) * bm;                  // queries in the last q-tile
@@ -125,7 +126,10 @@ constexpr size_t kQueueBytes = 256;  // 8 work-queue counters, padded
 // piece of each unit); more pieces run the separate merge kernel. So do calls whose items all run
 // at once, one per CU (one_round): a unit's last piece would merge alone at the end of the launch
 // (7-11 us) what the merge kernel spreads over the chip, and with no counters to clear and no
-// items to hand out they need no reset launch and no queues.
+// items to hand out they need no reset launch and no queues. us this way and with queues and
+// in-kernel merge, 5 heads x 3600 q in 3 pieces of 8 tiles 35.3, 37.1, of 48 88.5, 92.1, of 244
+// 375, 383; 3 heads in 5 pieces of 244 376, 406; 12 x 1560 in 3 of 24 54.7, 59.8. The long pieces
+// gain least, and over boxes (whose XCDs end apart) 5 x 3600 x 46800 was 1 % slower to 3.5 % faster.
 constexpr int kMaxFusedSplits = 8;
 
 struct Plan {
