@@ -181,7 +181,8 @@ def test_dmajor_tiles_equal_rows(lib, L, C, cap):
         assert torch.equal(v_out, v)
 
 
-@pytest.mark.parametrize("C,L", [(256, 2061), (640, 2061), (1024, 4173), (3072, 2061), (3072, 4173),
+@pytest.mark.parametrize("C,L", [(256, 2061), (640, 2061), (1024, 4173), (1536, 4173), (2048, 2061),
+                                 (2560, 2061), (3072, 2061), (3072, 4173),
                                  (3584, 2173), (4096, 2061), (4224, 2061), (4608, 4173),
                                  (5120, 2061), (5120, 4173), (3584, 6205), (4224, 6205),
                                  (5120, 6205)])
